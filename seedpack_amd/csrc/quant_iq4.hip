@@ -18,40 +18,38 @@ constexpr float GROUP_MAX_EPS = 1e-15f;
 // kvalues_iq4nl (ggml-common.h:1120)
 __constant__ const int8_t KVALUES[16] = {-127, -104, -83, -65, -49, -35, -22, -10, 1, 13, 25, 38, 53, 69, 89, 113};
 
-// best_index_int8(16, kvalues_iq4nl, x) -- ggml-quants.c:28-37: binary search, ties to the upper value.
-// The four halvings run unconditionally (the reference skips a step only on its [0, 1] range, where
-// the step cannot move: x > kvalues[0] there) and carry the values at both ends, so the final
-// nearest-of-two test needs no lookup. Levels 1-2 compare against constants; levels 3-4 read the
-// codebook from LDS (16 words on distinct banks): no per-lane global loads.
-struct Near {
-    int idx;     // best_index_int8's result
-    float val;   // kvalues_iq4nl[idx]
+// best_index_int8(16, kvalues_iq4nl, x) -- ggml-quants.c:28-37: the nearest value, ties to the upper
+// one. The midpoints of neighbouring values are whole or half numbers and the reference's distances
+// are exact near them, so the result depends on floor(2x) alone: a table over floor(2x), clamped to
+// the codebook's ends, holds it. One LDS read per weight and trial takes the place of the reference's
+// four halvings, the end tests and the nearest-of-two (about 30 instructions). NaN takes the last
+// value, as every comparison of the reference's search fails on it (the clamp's minimum comes first).
+constexpr int LUT_LO = -254, LUT_HI = 226, LUT_N = LUT_HI - LUT_LO + 1;
+struct Lut {
+    float val[LUT_N];      // kvalues_iq4nl[best_index]
+    uint8_t idx[LUT_N];
 };
-__device__ __forceinline__ Near nearest_iq4(const float* __restrict__ kv, float x) {
-    int lo = 0, hi = 15;
-    float vlo = (float)KVALUES[0], vhi = (float)KVALUES[15];
-    // level 1: mid 7
-    const bool c1 = x < (float)KVALUES[7];
-    if (c1) { hi = 7; vhi = (float)KVALUES[7]; } else { lo = 7; vlo = (float)KVALUES[7]; }
-    // level 2: mid 3 or 11
-    const float v2 = c1 ? (float)KVALUES[3] : (float)KVALUES[11];
-    const int m2 = c1 ? 3 : 11;
-    if (x < v2) { hi = m2; vhi = v2; } else { lo = m2; vlo = v2; }
+// filled by the workgroup's threads; the index at k = floor(2x) is the count of midpoints <= k / 2
+__device__ __forceinline__ void fill_lut(Lut& t) {
+    for (int i = threadIdx.x; i < LUT_N; i += WG) {
+        int n = 0;
 #pragma unroll
-    for (int it = 0; it < 2; ++it) {
-        const int mid = (lo + hi) >> 1;
-        const float v = kv[mid];
-        if (x < v) { hi = mid; vhi = v; } else { lo = mid; vlo = v; }
+        for (int j = 0; j < 15; ++j) n += i + LUT_LO >= KVALUES[j] + KVALUES[j + 1] ? 1 : 0;
+        t.idx[i] = (uint8_t)n;
+        t.val[i] = (float)KVALUES[n];
     }
-    Near r = x - vlo < vhi - x ? Near{lo, vlo} : Near{hi, vhi};
-    if (x >= (float)KVALUES[15]) r = Near{15, (float)KVALUES[15]};
-    if (x <= (float)KVALUES[0]) r = Near{0, (float)KVALUES[0]};
-    return r;
 }
-__device__ __forceinline__ int best_index(const float* __restrict__ kv, float x) { return nearest_iq4(kv, x).idx; }
+// the table's entry for x, from x2 = 2x
+__device__ __forceinline__ int lut_at(float x2) {
+    const float c = fmaxf(fminf(x2, (float)LUT_HI), (float)LUT_LO);
+    int k;
+    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(k) : "v"(c));
+    return k - LUT_LO;
+}
+__device__ __forceinline__ int best_index(const Lut& t, float x2) { return t.idx[lut_at(x2)]; }
 
 // scale search of one 32-weight block (ggml-quants.c:4962-5010, ntry = 7); returns the block scale
-__device__ __forceinline__ float block_scale(const float* __restrict__ kv, const float (&x)[32], const float (&w)[32]) {
+__device__ __forceinline__ float block_scale(const Lut& t, const float (&x)[32], const float (&w)[32]) {
     float amax = 0, max = 0;
 #pragma unroll
     for (int j = 0; j < 32; ++j) {
@@ -61,10 +59,11 @@ __device__ __forceinline__ float block_scale(const float* __restrict__ kv, const
     if (amax < GROUP_MAX_EPS) return 0.f;
     float d = -max / (float)KVALUES[0];
     float id = 1 / d;
+    float id2 = 2 * id;                // (2 id) x is 2 (id x); amax bounds id, so it is finite
     float sumqx = 0, sumq2 = 0;
 #pragma unroll
     for (int j = 0; j < 32; ++j) {
-        const float q = nearest_iq4(kv, id * x[j]).val;
+        const float q = t.val[lut_at(id2 * x[j])];
         sumqx += w[j] * q * x[j];
         sumq2 += w[j] * q * q;
     }
@@ -72,10 +71,11 @@ __device__ __forceinline__ float block_scale(const float* __restrict__ kv, const
     float best = d * sumqx;
     for (int itry = -7; itry <= 7; ++itry) {
         id = (float)(itry + KVALUES[0]) / max;
+        id2 = 2 * id;
         sumqx = sumq2 = 0;
 #pragma unroll
         for (int j = 0; j < 32; ++j) {
-            const float q = nearest_iq4(kv, id * x[j]).val;
+            const float q = t.val[lut_at(id2 * x[j])];
             sumqx += w[j] * q * x[j];
             sumq2 += w[j] * q * q;
         }
@@ -91,8 +91,8 @@ __device__ __forceinline__ float block_scale(const float* __restrict__ kv, const
 __global__ __launch_bounds__(WG) void k_iq4_nl(const void* __restrict__ src, int kind, uint8_t* __restrict__ dst,
                                                int64_t nblocks, int64_t bpr, const float* __restrict__ imx) {
     __shared__ __align__(16) uint16_t tile[WG * 18 / 2];
-    __shared__ float kv[16];
-    if (threadIdx.x < 16) kv[threadIdx.x] = (float)KVALUES[threadIdx.x];
+    __shared__ Lut lut;
+    fill_lut(lut);
     __syncthreads();
     const int64_t b0 = (int64_t)blockIdx.x * WG;
     const int64_t b = b0 + threadIdx.x;
@@ -112,14 +112,14 @@ __global__ __launch_bounds__(WG) void k_iq4_nl(const void* __restrict__ src, int
 #pragma unroll
             for (int j = 0; j < 32; ++j) w[j] = x[j] * x[j];
         }
-        const float d = block_scale(kv, x, w);
+        const float d = block_scale(lut, x, w);
         const float id = d != 0.f ? 1 / d : 0.f;
         TileOut o{tile + threadIdx.x * 9};
         o.put16(0, f32_to_f16(d));
 #pragma unroll
         for (int j = 0; j < 16; j += 2) {
-            const uint32_t b0_ = best_index(kv, id * x[j]) | (best_index(kv, id * x[16 + j]) << 4);
-            const uint32_t b1_ = best_index(kv, id * x[j + 1]) | (best_index(kv, id * x[17 + j]) << 4);
+            const uint32_t b0_ = best_index(lut, 2 * (id * x[j])) | (best_index(lut, 2 * (id * x[16 + j])) << 4);
+            const uint32_t b1_ = best_index(lut, 2 * (id * x[j + 1])) | (best_index(lut, 2 * (id * x[17 + j])) << 4);
             o.put2(2 + j, b0_, b1_);
         }
     }
@@ -135,8 +135,8 @@ __global__ __launch_bounds__(WG) void k_iq4_xs(const void* __restrict__ src, int
     __shared__ __align__(16) uint8_t ltile[SBW * 256];
     __shared__ __align__(16) uint16_t otile[SBW * 136 / 2];
     __shared__ int lsc[SBW][G];
-    __shared__ float kv[16];
-    if (threadIdx.x < 16) kv[threadIdx.x] = (float)KVALUES[threadIdx.x];
+    __shared__ Lut lut;
+    fill_lut(lut);
     __syncthreads();
     const int lsb = threadIdx.x / G, sub = threadIdx.x % G;
     const int64_t sb0 = (int64_t)blockIdx.x * SBW;
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(WG) void k_iq4_xs(const void* __restrict__ src, int
 #pragma unroll
         for (int j = 0; j < 32; ++j) w[j] = sq[j];
     }
-    const float scale = block_scale(kv, x, w);
+    const float scale = block_scale(lut, x, w);
     // the scale with the largest magnitude (first one on ties), then the super-scale
     float max_scale = 0, amax_scale = 0;
 #pragma unroll
@@ -185,8 +185,8 @@ __global__ __launch_bounds__(WG) void k_iq4_xs(const void* __restrict__ src, int
     uint32_t* lt = reinterpret_cast<uint32_t*>(ltile + lsb * 256 + sub * 32);
 #pragma unroll
     for (int j = 0; j < 32; j += 4)
-        lt[j / 4] = (uint32_t)best_index(kv, idl * x[j]) | ((uint32_t)best_index(kv, idl * x[j + 1]) << 8) |
-                    ((uint32_t)best_index(kv, idl * x[j + 2]) << 16) | ((uint32_t)best_index(kv, idl * x[j + 3]) << 24);
+        lt[j / 4] = (uint32_t)best_index(lut, 2 * (idl * x[j])) | ((uint32_t)best_index(lut, 2 * (idl * x[j + 1])) << 8) |
+                    ((uint32_t)best_index(lut, 2 * (idl * x[j + 2])) << 16) | ((uint32_t)best_index(lut, 2 * (idl * x[j + 3])) << 24);
     lsc[lsb][sub] = l + 32;
     __syncthreads();
     if (active && sub == 0) {

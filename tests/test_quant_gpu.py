@@ -229,3 +229,27 @@ def test_blocking_waits_give_the_same_bytes(gq):
         dev.set_blocking_waits(prev)
     assert dev.set_blocking_waits(prev) is False
     assert hip(gq, 12, x, imx).tobytes() == want
+
+
+@pytest.mark.parametrize("use_imx", [True, False])
+@pytest.mark.parametrize("t", [20, 23])
+def test_iq4_at_codebook_midpoints(gq, t, use_imx):
+    """the codebook table of the IQ4 types at its edges: weights that a trial scales onto every midpoint of
+    neighbouring codes, a float to each side of it, and the codebook's ends; sub-blocks of zeros and of
+    tiny weights beside them"""
+    kv = np.array([-127, -104, -83, -65, -49, -35, -22, -10, 1, 13, 25, 38, 53, 69, 89, 113], np.float32)
+    mid = (kv[1:] + kv[:-1]) / 2
+    vals = np.concatenate([mid, np.nextafter(mid, np.float32(-1e9)), np.nextafter(mid, np.float32(1e9)), kv[1:],
+                           np.float32([113.5, -126.5, 0.0, -0.0, 1e-30])]).astype(np.float32)
+    g = np.random.Generator(np.random.PCG64(20 + t))
+    x = g.choice(vals, size=(24, 256)).reshape(24, 8, 32)
+    x[:, :, 0] = -127                      # the block's largest: trial 0 scales by exactly 2^10
+    x[3, 2] = 0
+    x[5] = 0
+    x[7, 1] *= np.float32(2.0 ** -60)
+    x = (x * np.float32(2.0 ** -10)).reshape(24, 256)
+    imx = g.lognormal(0, 1, 256).astype(np.float32) if use_imx else None
+    got = gq.quantize_tensors(t, [(x.reshape(-1), 256)], [imx])[0]
+    want = quants.quantize(t, x, imx)
+    bad = np.flatnonzero(got != want)
+    assert bad.size == 0, f"{bad.size} bytes differ, first at {bad[:8]}"
