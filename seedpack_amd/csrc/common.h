@@ -128,6 +128,7 @@ struct TileOut {
         base[off >> 1] = (uint16_t)((lo & 0xffu) | ((hi & 0xffu) << 8));
     }
     __device__ __forceinline__ void put16(int off, uint32_t v) const { base[off >> 1] = (uint16_t)v; }
+    __device__ __forceinline__ void put4(int off, uint32_t v) const { put16(off, v & 0xffffu); put16(off + 2, v >> 16); }
 };
 
 // Copies `nbytes` (even) from an LDS tile to global memory at dst (2-byte aligned), using every

@@ -10,8 +10,8 @@
 // its terms to the running sum it receives from lane g-1 (a shuffle per hand-off), so the order is
 // the reference's. Sub-block results reach every lane of the group by shuffles; each lane repeats
 // the small super-block level searches (identical inputs, identical result), requantizes its own
-// sub-block, and parks its level values in LDS. Lane 0 of the group then packs the block bytes
-// into an LDS tile that the workgroup stores with coalesced dword writes.
+// sub-block, and parks its level values in LDS. The group's lanes then pack the block, each its share
+// of the words, into an LDS tile that the workgroup stores with coalesced dword writes.
 #include "common.h"
 #include "launch.h"
 #include "search.h"
@@ -212,36 +212,23 @@ struct Q45K {
             }
         }
     }
-    __device__ __forceinline__ static void pack(const KHeader& h, const uint8_t* L, TileOut o) {
-        o.put16(0, h.d);
-        o.put16(2, h.dmin);
+    __device__ __forceinline__ static void pack(const KHeader& h, const uint32_t* L, TileOut o, int sub) {
+        if (sub == 0) {
+            o.put16(0, h.d);
+            o.put16(2, h.dmin);
 #pragma unroll
-        for (int j = 0; j < 12; j += 2) o.put2(4 + j, h.sc[j], h.sc[j + 1]);
-        if (NMAX == 15) {   // Q4_K: qs[128] at 16
-            for (int j = 0; j < 256; j += 64)
-                for (int l = 0; l < 32; l += 2)
-                    o.put2(16 + j / 2 + l, L[j + l] | (L[j + l + 32] << 4), L[j + l + 1] | (L[j + l + 33] << 4));
-        } else {            // Q5_K: qh[32] at 16, qs[128] at 48 (ggml-quants.c:1711-1729)
-            for (int j = 0; j < 32; j += 2) {
-                uint32_t qh[2];
-                for (int k = 0; k < 2; ++k) {
-                    uint32_t v = 0;
-                    for (int n = 0; n < 4; ++n)
-                        v |= ((L[64 * n + j + k] > 15 ? 1u : 0u) << (2 * n)) | ((L[64 * n + j + k + 32] > 15 ? 2u : 0u) << (2 * n));
-                    qh[k] = v;
-                }
-                o.put2(16 + j, qh[0], qh[1]);
-            }
-            for (int n = 0; n < 256; n += 64)
-                for (int j = 0; j < 32; j += 2) {
-                    uint32_t q[2];
-                    for (int k = 0; k < 2; ++k) {
-                        const uint32_t l1 = L[n + j + k], l2 = L[n + j + k + 32];
-                        q[k] = ((l1 > 15 ? l1 - 16 : l1) | ((l2 > 15 ? l2 - 16 : l2) << 4)) & 0xff;
-                    }
-                    o.put2(48 + n / 2 + j, q[0], q[1]);
-                }
+            for (int j = 0; j < 12; j += 2) o.put2(4 + j, h.sc[j], h.sc[j + 1]);
         }
+        constexpr int QS = NMAX == 15 ? 16 : 48;
+        if (NMAX == 31) {   // Q5_K: qh[32] at 16, qs[128] at 48 (ggml-quants.c:1711-1729): bits 2n, 2n + 1
+            uint32_t v = 0;
+#pragma unroll
+            for (int n = 0; n < 8; ++n) v |= ((L[8 * n + sub] >> 4) & 0x01010101u) << n;
+            o.put4(16 + 4 * sub, v);
+        }
+#pragma unroll
+        for (int n = 0; n < 4; ++n)     // low nibbles: levels of 32 weights, then of the next 32 above them
+            o.put4(QS + 32 * n + 4 * sub, (L[16 * n + sub] & 0x0f0f0f0fu) | ((L[16 * n + 8 + sub] & 0x0f0f0f0fu) << 4));
     }
 };
 
@@ -362,18 +349,15 @@ struct Q2K {
             }
         }
     }
-    __device__ __forceinline__ static void pack(const KHeader& h, const uint8_t* L, TileOut o) {
+    __device__ __forceinline__ static void pack(const KHeader& h, const uint32_t* L, TileOut o, int sub) {
+        if (sub == 0) {
 #pragma unroll
-        for (int j = 0; j < 16; j += 2) o.put2(j, h.sc[j], h.sc[j + 1]);
-        for (int j = 0; j < 256; j += 128)
-            for (int l = 0; l < 32; l += 2) {
-                uint32_t q[2];
-                for (int k = 0; k < 2; ++k)
-                    q[k] = (L[j + l + k] | (L[j + l + k + 32] << 2) | (L[j + l + k + 64] << 4) | (L[j + l + k + 96] << 6)) & 0xff;
-                o.put2(16 + j / 4 + l, q[0], q[1]);
-            }
-        o.put16(80, h.d);
-        o.put16(82, h.dmin);
+            for (int j = 0; j < 16; j += 2) o.put2(j, h.sc[j], h.sc[j + 1]);
+            o.put16(80, h.d);
+            o.put16(82, h.dmin);
+        }
+        const uint32_t* p = L + 32 * (sub / 8) + sub % 8;
+        o.put4(16 + 4 * sub, p[0] | (p[8] << 2) | (p[16] << 4) | (p[24] << 6));
     }
 };
 
@@ -547,29 +531,23 @@ struct Q3K {
             }
         }
     }
-    __device__ __forceinline__ static void pack(const KHeader& h, const uint8_t* L, TileOut o) {
+    __device__ __forceinline__ static void pack(const KHeader& h, const uint32_t* L, TileOut o, int sub) {
         // hmask[32] at 0, qs[64] at 32, scales[12] at 96, d at 108 (ggml-quants.c:1410-1435). Levels are
         // 0..7: bit 2 goes to hmask (bit k of byte m for level 32k+m) and the low two bits to qs.
-        for (int m = 0; m < 32; m += 2) {
-            uint32_t hb[2];
-            for (int k2 = 0; k2 < 2; ++k2) {
-                uint32_t v = 0;
-                for (int k = 0; k < 8; ++k) v |= (L[32 * k + m + k2] > 3 ? 1u : 0u) << k;
-                hb[k2] = v;
-            }
-            o.put2(m, hb[0], hb[1]);
-        }
-        for (int j = 0; j < 256; j += 128)
-            for (int l = 0; l < 32; l += 2) {
-                uint32_t q[2];
-                for (int k = 0; k < 2; ++k)
-                    q[k] = ((L[j + l + k] & 3) | ((L[j + l + k + 32] & 3) << 2) | ((L[j + l + k + 64] & 3) << 4) |
-                            ((L[j + l + k + 96] & 3) << 6)) & 0xff;
-                o.put2(32 + j / 4 + l, q[0], q[1]);
-            }
+        if (sub < 8) {
+            uint32_t v = 0;
 #pragma unroll
-        for (int j = 0; j < 12; j += 2) o.put2(96 + j, h.sc[j], h.sc[j + 1]);
-        o.put16(108, h.d);
+            for (int k = 0; k < 8; ++k) v |= ((L[8 * k + sub] >> 2) & 0x01010101u) << k;
+            o.put4(4 * sub, v);
+        }
+        const uint32_t* p = L + 32 * (sub / 8) + sub % 8;
+        o.put4(32 + 4 * sub, (p[0] & 0x03030303u) | ((p[8] & 0x03030303u) << 2) | ((p[16] & 0x03030303u) << 4) |
+                                 ((p[24] & 0x03030303u) << 6));
+        if (sub == 15) {
+#pragma unroll
+            for (int j = 0; j < 12; j += 2) o.put2(96 + j, h.sc[j], h.sc[j + 1]);
+            o.put16(108, h.d);
+        }
     }
 };
 
@@ -626,31 +604,22 @@ struct Q6K {
             }
         }
     }
-    __device__ __forceinline__ static void pack(const KHeader& h, const uint8_t* L, TileOut o) {
-        // ql[128] at 0, qh[64] at 128, scales[16] at 192, d at 208 (ggml-quants.c:1922-1935)
-        if (h.zero) {
-            for (int j = 0; j < 210; j += 2) o.put16(j, 0);
-            return;
-        }
-        for (int j = 0; j < 256; j += 128) {
-            for (int l = 0; l < 32; l += 2) {
-                uint32_t a[2], b[2], c[2];
-                for (int k = 0; k < 2; ++k) {
-                    const uint32_t q1 = L[j + l + k + 0] & 0xF, q2 = L[j + l + k + 32] & 0xF;
-                    const uint32_t q3 = L[j + l + k + 64] & 0xF, q4 = L[j + l + k + 96] & 0xF;
-                    a[k] = (q1 | (q3 << 4)) & 0xff;
-                    b[k] = (q2 | (q4 << 4)) & 0xff;
-                    c[k] = ((L[j + l + k] >> 4) | ((L[j + l + k + 32] >> 4) << 2) | ((L[j + l + k + 64] >> 4) << 4) |
-                            ((L[j + l + k + 96] >> 4) << 6)) & 0xff;
-                }
-                o.put2(j / 2 + l, a[0], a[1]);
-                o.put2(j / 2 + l + 32, b[0], b[1]);
-                o.put2(128 + j / 4 + l, c[0], c[1]);
-            }
-        }
+    __device__ __forceinline__ static void pack(const KHeader& h, const uint32_t* L, TileOut o, int sub) {
+        // ql[128] at 0, qh[64] at 128, scales[16] at 192, d at 208 (ggml-quants.c:1922-1935); an all-zero
+        // super-block is all zero bytes
+        const int half = sub / 8, l = sub % 8;
+        const uint32_t keep = h.zero ? 0u : ~0u;
+        const uint32_t* p = L + 32 * half + l;
+        const uint32_t q1 = p[0] & keep, q2 = p[8] & keep, q3 = p[16] & keep, q4 = p[24] & keep;
+        o.put4(64 * half + 4 * l, (q1 & 0x0f0f0f0fu) | ((q3 & 0x0f0f0f0fu) << 4));
+        o.put4(64 * half + 4 * l + 32, (q2 & 0x0f0f0f0fu) | ((q4 & 0x0f0f0f0fu) << 4));
+        o.put4(128 + 32 * half + 4 * l, ((q1 >> 4) & 0x03030303u) | (((q2 >> 4) & 0x03030303u) << 2) |
+                                            (((q3 >> 4) & 0x03030303u) << 4) | (((q4 >> 4) & 0x03030303u) << 6));
+        if (sub == 0) {
 #pragma unroll
-        for (int j = 0; j < 16; j += 2) o.put2(192 + j, h.sc[j], h.sc[j + 1]);
-        o.put16(208, h.d);
+            for (int j = 0; j < 16; j += 2) o.put2(192 + j, h.zero ? 0u : h.sc[j], h.zero ? 0u : h.sc[j + 1]);
+            o.put16(208, h.d);
+        }
     }
 };
 
@@ -713,7 +682,10 @@ __global__ __launch_bounds__(WG) void k_kquant(const void* __restrict__ src, int
     Op::requant(x, h, ginfo[lsb][sub], L);
     park_levels<SUB>(ltile + lsb * 256 + sub * SUB, L);
     __syncthreads();
-    if (active && sub == 0) Op::pack(h, ltile + lsb * 256, TileOut{otile + lsb * (Op::BS / 2)});
+    // each lane of the group packs its share of the block, four levels (one word of the tile) at a time:
+    // packed by one lane, the block's 256 levels cost the wave up to a third of its instructions (Q6_K on
+    // 151936 x 1024: 994 us, 732 us shared out; Q4_K on 12288 x 4096: 736 and 714 us)
+    if (active) Op::pack(h, reinterpret_cast<const uint32_t*>(ltile + lsb * 256), TileOut{otile + lsb * (Op::BS / 2)}, sub);
     __syncthreads();
     const int nb = (int)(nsb - sb0 < SBW ? nsb - sb0 : SBW);
     store_tile(otile, dst + sb0 * Op::BS, nb * Op::BS);
