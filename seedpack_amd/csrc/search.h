@@ -12,9 +12,58 @@ namespace spa {
 
 constexpr float GROUP_MAX_EPS = 1e-15f;   // ggml-quants.c:20
 
+// whether any of x is infinite or NaN (the largest exponent of all, signs shifted out)
+template <int N>
+__device__ __forceinline__ bool not_finite(const float (&x)[N]) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) m = tmax(m, __float_as_uint(x[i]) << 1);
+    return m >= 0xff000000u;
+}
+
+// The trial scales of make_qx_quants, its start (is == 0) first: the scale of the best one and, in
+// best_iscale, the inverse scale that gives its levels.
+// FLOAT: the level nearest_int(v) clamped is formed as rint(v) clamped, both in float: the same number
+// for every |v| < 2^22, and here |v| <= nmax + 1 as long as the weights are finite (a level may be -0.0
+// instead of 0, which changes no sum: sums start at +0.0 and adding either zero keeps them). Three
+// instructions per weight and trial instead of six. The others follow the C expressions.
+template <int N, bool QW, bool FLOAT>
+__device__ __forceinline__ float qx_trials(int nmax, const float (&x)[N], const float (&qw)[N], float max, float& best_iscale) {
+    const float lo = (float)(-nmax), hi = (float)(nmax - 1);
+    float scale = 0, best = 0;
+    for (int k = -10; k <= 9; ++k) {
+        const bool first = k == -10;
+        const int is = first ? 0 : k;
+        if (!first && is == 0) continue;
+        const float isc = first ? lo / max : -((float)nmax + 0.1f * (float)is) / max;
+        float slx = 0, sl2 = 0;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            float l;
+            if constexpr (FLOAT) l = __builtin_amdgcn_fmed3f(rintf(isc * x[i]), lo, hi);
+            else l = (float)tmax(-nmax, tmin(nmax - 1, nearest_int(isc * x[i])));
+            const float w = QW ? qw[i] : x[i] * x[i];
+            slx += w * x[i] * l;
+            sl2 += w * l * l;
+        }
+        if (first) {
+            best_iscale = isc;
+            scale = sl2 != 0.f ? slx / sl2 : 0.0f;
+            best = scale * slx;
+        } else if (sl2 > 0 && slx * slx > best * sl2) {
+            best_iscale = isc;
+            scale = slx / sl2;
+            best = scale * slx;
+        }
+    }
+    return scale;
+}
+
 // make_qx_quants(n, nmax, x, L, rmse_type = 1, qw) -- ggml-quants.c:628-695.
 // QW = true: w = qw[i]; QW = false (qw == NULL): w = x[i]*x[i].
 // L[i] receives nmax + clamp(l, -nmax, nmax-1).
+// Bound by VALU issue (19 trials of N weights). The float levels (see qx_trials) took Q6_K with the
+// importance matrix on 151936 x 1024 from 732 us to 630 us.
 template <int N, bool QW>
 __device__ __forceinline__ float make_qx_quants(int nmax, const float (&x)[N], const float (&qw)[N], int (&L)[N]) {
     float max = 0, amax = 0;
@@ -28,37 +77,9 @@ __device__ __forceinline__ float make_qx_quants(int nmax, const float (&x)[N], c
         for (int i = 0; i < N; ++i) L[i] = 0;
         return 0.f;
     }
-    float iscale = (float)(-nmax) / max;
-    float sumlx = 0, suml2 = 0;
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        int l = nearest_int(iscale * x[i]);
-        l = tmax(-nmax, tmin(nmax - 1, l));
-        const float w = QW ? qw[i] : x[i] * x[i];
-        sumlx += w * x[i] * (float)l;
-        suml2 += w * (float)l * (float)l;
-    }
-    float scale = suml2 != 0.f ? sumlx / suml2 : 0.0f;
-    float best = scale * sumlx;
-    float best_iscale = iscale;
-    for (int is = -9; is <= 9; ++is) {
-        if (is == 0) continue;
-        const float isc = -((float)nmax + 0.1f * (float)is) / max;
-        float slx = 0, sl2 = 0;
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            int l = nearest_int(isc * x[i]);
-            l = tmax(-nmax, tmin(nmax - 1, l));
-            const float w = QW ? qw[i] : x[i] * x[i];
-            slx += w * x[i] * (float)l;
-            sl2 += w * (float)l * (float)l;
-        }
-        if (sl2 > 0 && slx * slx > best * sl2) {
-            best_iscale = isc;
-            scale = slx / sl2;
-            best = scale * slx;
-        }
-    }
+    float best_iscale, scale;
+    if (__ballot(not_finite(x))) scale = qx_trials<N, QW, false>(nmax, x, qw, max, best_iscale);
+    else scale = qx_trials<N, QW, true>(nmax, x, qw, max, best_iscale);
     // L is a pure function of the winning iscale, so it is produced once here.
 #pragma unroll
     for (int i = 0; i < N; ++i) {

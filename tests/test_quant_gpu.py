@@ -253,3 +253,23 @@ def test_iq4_at_codebook_midpoints(gq, t, use_imx):
     want = quants.quantize(t, x, imx)
     bad = np.flatnonzero(got != want)
     assert bad.size == 0, f"{bad.size} bytes differ, first at {bad[:8]}"
+
+
+@pytest.mark.parametrize("use_imx", [True, False])
+@pytest.mark.parametrize("t", [2, 6, 11, 14, 20, 23])
+def test_infinite_and_nan_weights(gq, t, use_imx):
+    """blocks with infinities, NaN and the largest finite values beside finite ones, and a zero
+    importance: the trial searches take the same decisions as the C expressions there"""
+    g = np.random.Generator(np.random.PCG64(5))
+    x = (g.standard_normal((16, 512)) * 0.02).astype(np.float32)
+    x[1, 5], x[2, 300], x[3, 7] = np.inf, -np.inf, np.nan
+    x[4, 100:140] = np.inf
+    x[5, 40:42] = np.inf, -np.inf
+    x[6, 17:19] = 3e38, -3e38
+    imx = g.lognormal(0, 1, 512).astype(np.float32)
+    imx[17] = 0
+    imx = imx if use_imx else None
+    got = gq.quantize_tensors(t, [(x.reshape(-1), 512)], [imx])[0]
+    with np.errstate(all="ignore"):
+        want = quants.quantize(t, x, imx)
+    assert np.array_equal(got, want)
