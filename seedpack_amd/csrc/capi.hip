@@ -196,7 +196,8 @@ int spa_quantize(int t, int variant, const void* src, int src_kind, int64_t nrow
         case 2: case 3: case 6: case 7: case 8: case 42: return spa::launch_legacy(a);
         case 10: case 11: case 12: case 13: case 14: return spa::launch_kquant(a);
         case 20: case 23: return spa::launch_iq4(a);
-        default: return spa::launch_iqgrid(a);
+        case 19: case 29: return spa::launch_iq1(a);
+        default: return spa::launch_lattice(a);
     }
 }
 

@@ -8,8 +8,8 @@ namespace spa {
 
 struct IqDeviceTable {
     const uint8_t* grid;      // size x (8 or 4) coordinate values 2l+1
-    const int32_t* map;       // level index -> grid point, or -1 - (offset << 9 | length) of its list in nb
-    const uint16_t* nb;       // neighbour lists: count, then grid point indices
+    const int32_t* map;       // level index -> grid point, or -1 - (offset / 8 << 9 | length) of its list in nb
+    const uint16_t* nb;       // neighbour lists: grid point indices, each padded to a multiple of 8 with `size`
     int size;
 };
 

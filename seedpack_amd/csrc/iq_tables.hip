@@ -110,22 +110,30 @@ struct DevTable {
     hipEvent_t ready = nullptr;
 };
 DevTable g_dev[MAXDEV][6];
-// the device form of each table's map (list lengths packed beside their offsets), built once per
-// process and kept: queued copies read it after the call that queued them has returned
+// the device form of each table's map and lists: every list starts on a multiple of 8 entries (16 bytes:
+// the kernels read 4 or 8 at a time; the rest of its last 8 names the point after the codebook's last), its
+// offset and length packed in the map. Built once per process and kept: queued copies read it after the
+// call that queued them has returned.
 std::once_flag g_dm_once[6];
 std::vector<int32_t> g_dm[6];
+std::vector<uint16_t> g_dn[6];
 int g_dm_err[6];
 
 const std::vector<int32_t>& device_map(int idx) {
     std::call_once(g_dm_once[idx], [idx] {
         const Host& h = host_table(idx);
         std::vector<int32_t>& dm = g_dm[idx];
+        std::vector<uint16_t>& dn = g_dn[idx];
         dm.resize(h.map.size());
+        dn.reserve(2 * h.nb.size());
         for (size_t i = 0; i < h.map.size(); ++i) {
             const int32_t v = h.map[i];
             if (v >= 0) { dm[i] = v; continue; }
-            const uint32_t off = (uint32_t)(-v - 1), len = h.nb[off];
+            const uint16_t* list = &h.nb[(size_t)(-v - 1)];
+            const uint32_t off = (uint32_t)(dn.size() / 8), len = list[0];
             if (off >= (1u << 22) || len == 0 || len >= 512) { g_dm_err[idx] = 1; return; }
+            dn.insert(dn.end(), list + 1, list + 1 + len);
+            while (dn.size() % 8) dn.push_back((uint16_t)kSpecs[idx].size);
             dm[i] = -1 - (int32_t)((off << 9) | len);
         }
     });
@@ -155,11 +163,12 @@ int iq_device_table(int idx, IqDeviceTable* out, hipStream_t stream) {
     const Host& h = host_table(idx);
     const std::vector<int32_t>& dm = device_map(idx);
     if (g_dm_err[idx]) return fail(SPA_ERR_ARG, "iq table %d: a neighbour list does not fit the packed map", idx);
+    const std::vector<uint16_t>& dn = g_dn[idx];
     std::lock_guard<std::mutex> lk(g_dev_mu);
     DevTable& d = g_dev[dev][idx];
     if (!d.t.grid) {
         const size_t og = 0, om = align256(h.grid.size()), on = om + align256(dm.size() * sizeof(int32_t));
-        const size_t total = on + h.nb.size() * sizeof(uint16_t);
+        const size_t total = on + dn.size() * sizeof(uint16_t);
         uint8_t* base = nullptr;
         hipEvent_t ev = nullptr;
         hipError_t e = hipMalloc((void**)&base, total);
@@ -168,7 +177,7 @@ int iq_device_table(int idx, IqDeviceTable* out, hipStream_t stream) {
         if (e == hipSuccess)
             e = hipMemcpyAsync(base + om, dm.data(), dm.size() * sizeof(int32_t), hipMemcpyHostToDevice, stream);
         if (e == hipSuccess)
-            e = hipMemcpyAsync(base + on, h.nb.data(), h.nb.size() * sizeof(uint16_t), hipMemcpyHostToDevice, stream);
+            e = hipMemcpyAsync(base + on, dn.data(), dn.size() * sizeof(uint16_t), hipMemcpyHostToDevice, stream);
         if (e == hipSuccess) e = hipEventRecord(ev, stream);
         if (e != hipSuccess) {
             // nothing is published: wait for whatever was queued, then release it

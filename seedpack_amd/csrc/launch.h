@@ -31,7 +31,8 @@ int type_bs(int type);
 int launch_legacy(const QuantArgs& a);   // Q4_0 Q4_1 Q5_0 Q5_1 Q8_0 Q2_0
 int launch_kquant(const QuantArgs& a);   // Q2_K Q3_K Q4_K Q5_K Q6_K
 int launch_iq4(const QuantArgs& a);      // IQ4_NL IQ4_XS
-int launch_iqgrid(const QuantArgs& a);   // IQ2_XXS IQ2_XS IQ2_S IQ3_XXS IQ3_S IQ1_S IQ1_M
+int launch_lattice(const QuantArgs& a);  // IQ2_XXS IQ2_XS IQ2_S IQ3_XXS IQ3_S
+int launch_iq1(const QuantArgs& a);      // IQ1_S IQ1_M
 
 // Sets the thread's last error message (printf-style) and returns `code`.
 int fail(int code, const char* fmt, ...);

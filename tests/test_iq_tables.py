@@ -51,3 +51,51 @@ def test_neighbour_lists_are_nearest_by_brute_force():
         levels = np.unique(d2)[:2]
         want = [j for d in levels for j in np.flatnonzero(d2 == d)]
         assert list(lst) == want
+
+
+@pytest.mark.parametrize("i, d, levels, l1, m2, p1, p2", [(0, 8, 3, 20, 128, 24, 144), (1, 8, 3, 20, 128, 24, 144),
+                                                          (3, 8, 3, 20, 128, 24, 144), (4, 4, 8, 16, 336, 24, 480),
+                                                          (5, 4, 8, 16, 336, 24, 480)])
+def test_spread_of_the_neighbour_lists(i, d, levels, l1, m2, p1, p2):
+    """the lattice quantizers' bounds (ListBound in csrc/quant_lattice.hip): sums over the coordinates of
+    |q - q'| and |q^2 - q'^2| between a list's first point and another, and between any two of its points, over
+    every list a rounded group can reach; and the 32-bit ranges that follow from them"""
+    grid, kmap, nbs = host_table(i)
+    pts = grid.reshape(-1, d).astype(np.int64)
+    bits = 2 if d == 8 else 3
+    top = np.zeros(4, np.int64)
+    for u in range(kmap.size):
+        lev = (u >> (bits * np.arange(d))) & ((1 << bits) - 1)
+        if lev.max() >= levels or kmap[u] >= 0:
+            continue
+        o = -int(kmap[u]) - 1
+        p = pts[nbs[o + 1:o + 1 + int(nbs[o])]]
+        q = p * p
+        top = np.maximum(top, [np.abs(p - p[0]).sum(1).max(), np.abs(q - q[0]).sum(1).max(),
+                               np.abs(p[:, None] - p[None]).sum(-1).max(), np.abs(q[:, None] - q[None]).sum(-1).max()])
+    assert (top <= [l1, m2, p1, p2]).all(), top
+    vmax = 1 << (23 if d == 8 else 22)
+    assert p2 * vmax < 1 << 31 and m2 * vmax < 1 << 31 and (pts * pts).sum(1).max() * vmax < 1 << 32
+
+
+def test_trial_scales_divide_exactly():
+    """the lattice quantizers' trial scales: num / max as one remainder step on num * (1 / max) in float32, for
+    every num of the types and a sample of mantissas that holds the ends of the range. The fused steps are
+    formed in float64: the remainder is exact there, and the last sum's rounding error decides its ties"""
+    f, d = np.float32, np.float64
+    nums = [f(5) + f(k) * f(0.1) for k in range(-9, 10)] + [f(15) + f(k) * f(0.2) for k in range(-15, 16)]
+    m = np.unique(np.concatenate([np.arange(4096), np.arange((1 << 23) - 4096, 1 << 23), np.arange(0, 1 << 23, 127)]))
+    mx = (m.astype(np.uint32) | np.uint32(0x3F800000)).view(f)
+    r = f(1) / mx
+    for num in nums:
+        q0 = num * r
+        rem = (d(num) - mx.astype(d) * q0.astype(d)).astype(f)
+        t = rem.astype(d) * r.astype(d)
+        s = q0.astype(d) + t
+        err = t - (s - q0.astype(d))                       # exact: |t| is far below |q0|
+        want = num / mx
+        # the exact sum s + err lies within half the gap to either neighbour of the quotient
+        up, dn = np.nextafter(want, f(9e9)).astype(d), np.nextafter(want, f(-9e9)).astype(d)
+        w = want.astype(d)
+        over, under = s - (w + up) / 2, s - (w + dn) / 2
+        assert ((over < 0) | ((over == 0) & (err <= 0))).all() and ((under > 0) | ((under == 0) & (err >= 0))).all()

@@ -273,3 +273,43 @@ def test_infinite_and_nan_weights(gq, t, use_imx):
     with np.errstate(all="ignore"):
         want = quants.quantize(t, x, imx)
     assert np.array_equal(got, want)
+
+
+def _lattice_edges(g):
+    """rows of 256 for the lattice searches: equal magnitudes (every list has ties), two magnitudes, unit and
+    zero importance, a huge weight where the importance is zero, sub-blocks scaled far down and up, zeros"""
+    x = (g.standard_t(5, size=(40, 256)) * 0.01).astype(np.float32)
+    imx = g.lognormal(0, 1, size=256).astype(np.float32)
+    imx[37], imx[200:204] = 0, 0
+    x[0] = 0.01 * np.sign(x[0])
+    x[1] = np.where(np.arange(256) % 3 == 0, 0.01, 0.003) * np.sign(x[1])
+    x[2] = np.round(x[2] * 500) / 500
+    x[3, 37] = 1e5
+    x[4, 37], x[4, 200] = -3e9, 1e30
+    x[5] *= np.float32(1e-19)
+    x[6] *= np.float32(1e-25)
+    x[7] *= np.float32(1e19)
+    x[8] *= np.repeat(np.float32([1, 1e-9, 1e-4, 1, 0, 1e-7, 1, 1e-14]), 32)
+    x[9, ::2] = 0
+    x[10] = np.abs(x[10])
+    x[11:16] = np.round(x[11:16] * 64) / 64
+    return x.astype(np.float32), imx
+
+
+@pytest.mark.parametrize("which", ["imatrix", "unit", "none"])
+@pytest.mark.parametrize("t", [16, 17, 18, 21, 22])
+def test_lattice_searches_at_ties_and_extremes(gq, t, which):
+    if which == "none" and t in NEED_IMX:
+        pytest.skip("the type needs an importance matrix")
+    x, imx = _lattice_edges(np.random.Generator(np.random.PCG64(900 + t)))
+    imx = {"imatrix": imx, "unit": np.ones(256, np.float32), "none": None}[which]
+    got = gq.quantize_tensors(t, [(x.reshape(-1), 256)], [imx])[0].reshape(len(x), -1)
+    compared = 0
+    for r in range(len(x)):
+        try:
+            want = np.asarray(quants.quantize(t, x[r:r + 1], imx))
+        except ValueError:                       # no listed point at a finite distance: the reference asserts
+            continue
+        assert np.array_equal(got[r], want), f"row {r} differs"
+        compared += 1
+    assert compared >= len(x) - 4
