@@ -22,6 +22,8 @@
 //     writes each symbol's (frequency << 16 | cumulative) word; the serial coder (one lane per
 //     segment, as the format requires) then streams those words;
 //   * decode: one lane per segment.
+#include <climits>
+
 #include "../../include/seedpack_amd.h"
 #include "common.h"
 #include "detmath.h"
@@ -436,9 +438,11 @@ __global__ __launch_bounds__(64) void k_enc(const SG* __restrict__ sg, int nseg,
 // more symbols (only symbols of fewer than 128 slots make one) holds the first and last of them with
 // the first one's cum and freq, first | (last - first) << 8 | cum << 16 | freq << 32, bit 63 set; a
 // slot past the first symbol is then found by binary search over the bucket's other symbols. Every
-// slot gets the symbol a full 2^15-entry lookup table gives; 3 KB per table instead of 32 KB.
+// slot gets the symbol a full 2^15-entry lookup table gives; 3.3 KB per table instead of 32 KB.
 // Contexts without a table (never coded) get a one-symbol table, reached only by damaged streams.
-constexpr int DT_BYTES = 3072;
+// Then what the decoder copies to LDS: each bucket's first symbol (256 u8), and the last 16 symbols up
+// to the last one coded: their cumulative frequencies (16 u16) and the first of them (u32).
+constexpr int DT_FIRST = 3072, DT_LAST16 = 3328, DT_BYTES = 3376;
 __device__ __forceinline__ int dec_sym(const uint8_t* dt, uint32_t slot, uint32_t& c0, uint32_t& f) {
     const uint64_t e = reinterpret_cast<const uint64_t*>(dt)[slot >> 7];
     if (!(e >> 63)) {
@@ -478,6 +482,8 @@ __global__ __launch_bounds__(256) void k_dtab(const uint32_t* __restrict__ cum, 
                                               uint8_t* __restrict__ dt) {
     __shared__ uint32_t ps[256];
     __shared__ uint32_t cs[257];
+    __shared__ int top;                  // the last symbol coded
+    if (threadIdx.x == 0) top = 0;
     const int t = remap[blockIdx.x];
     const uint32_t* c = cum + (size_t)(t < 0 ? 0 : t) * 257;
     uint8_t* o = dt + (size_t)blockIdx.x * DT_BYTES;
@@ -488,6 +494,7 @@ __global__ __launch_bounds__(256) void k_dtab(const uint32_t* __restrict__ cum, 
     const uint32_t fi = cs[i + 1] > cs[i] ? cs[i + 1] - cs[i] : 0u;
     ps[i] = cs[i] | (fi << 16);
     reinterpret_cast<uint32_t*>(o + 2048)[i] = ps[i];
+    if (fi) atomicMax(&top, i);
     // the symbol holding a slot: the last s <= 255 with cum[s] <= slot
     auto holder = [&](uint32_t slot) {
         int lo = 0, hi = 256;
@@ -512,143 +519,316 @@ __global__ __launch_bounds__(256) void k_dtab(const uint32_t* __restrict__ cum, 
             (1ull << 63);
     }
     reinterpret_cast<uint64_t*>(o)[i] = e;
+    o[DT_FIRST + i] = (uint8_t)first;
+    __syncthreads();
+    const int s16 = top > 15 ? top - 15 : 0;
+    if (i < 16) reinterpret_cast<uint16_t*>(o + DT_LAST16)[i] = (uint16_t)cs[s16 + i];
+    if (i == 16) *reinterpret_cast<uint32_t*>(o + DT_LAST16 + 32) = (uint32_t)s16;
 }
 
-// A lane's reader of its segment's bytes: a 16-byte window in registers refilled from the next
-// aligned 16-byte block, which is already loaded (its load issued when the window was last refilled),
-// so the coded stream is read once from HBM and its latency hides behind the decoding; blocks at or
-// past `lim` (the stream's length rounded up to 16 bytes) read as zeros.
+// A lane's reader of its segment's bytes: up to 64 bits in a register pair, the next byte on top, filled a
+// dword at a time from a 64-byte ring of the lane's own in LDS, the next dword already read from it. The
+// ring is topped up between weights with 16-byte blocks of the stream that were requested a top-up before
+// (so the stream is read once from HBM and its latency hides behind the decoding; no register with a load in
+// flight is moved in between). Blocks at or past `lim` (the stream's length rounded up to 16 bytes) read as
+// zeros.
 struct Reader {
     const uint4* p;
     const uint4* lim;
-    uint4 w, nx;                                 // w.x holds the current dword; consumed dwords shift out
-    int left, b;                                 // dwords left in the window, byte index in w.x
-    __device__ __forceinline__ uint4 fetch() {
-        const uint4 v = p < lim ? *p : make_uint4(0u, 0u, 0u, 0u);
+    uint4 blk;                                   // the next block, in flight
+    uint4* ring;                                 // this lane's 4 blocks
+    uint32_t pos, end;                           // bytes taken from the ring, written to it
+    uint32_t nd;                                 // the ring's dword at pos
+    uint64_t q;                                  // bits read and not yet used, at the top
+    int nb;                                      // their number
+    __device__ __forceinline__ void request() {
+        blk = p < lim ? *p : make_uint4(0u, 0u, 0u, 0u);
         ++p;
-        return v;
     }
-    __device__ __forceinline__ void next_dword() {
-        w.x = w.y;
-        w.y = w.z;
-        w.z = w.w;
-        if (--left == 0) {
-            w = nx;
-            nx = fetch();
-            left = 4;
+    // more than 48 bytes in the ring afterwards: four weights take at most 24, and the dword after them
+    __device__ __forceinline__ void top_up() {
+        while ((int)(end - pos) <= 48) {
+            ring[(end >> 4) & 3] = blk;
+            end += 16;
+            request();
         }
     }
-    __device__ __forceinline__ void start(const uint8_t* base, uint64_t off, uint64_t nblocks) {
+    __device__ __forceinline__ void peek() { nd = reinterpret_cast<const uint32_t*>(ring)[(pos >> 2) & 15]; }
+    // 32 bits more (at most 32 before)
+    __device__ __forceinline__ void fill() {
+        q |= (uint64_t)__builtin_bswap32(nd) << (32 - nb);
+        nb += 32;
+        pos += 4;
+    }
+    __device__ __forceinline__ void drop(int bits) {
+        q <<= bits;
+        nb -= bits;
+    }
+    __device__ __forceinline__ void start(const uint8_t* base, uint64_t off, uint64_t nblocks, uint4* lane_ring) {
         p = reinterpret_cast<const uint4*>(base) + (off >> 4);
         lim = reinterpret_cast<const uint4*>(base) + nblocks;
-        w = fetch();
-        nx = fetch();
-        left = 4;
-        for (int q = (int)((off >> 2) & 3); q > 0; --q) next_dword();
-        b = (int)(off & 3);
-    }
-    __device__ __forceinline__ uint32_t byte() {
-        const uint32_t v = (w.x >> (8 * b)) & 0xFFu;
-        if (++b == 4) {
-            b = 0;
-            next_dword();
-        }
-        return v;
+        ring = lane_ring;
+        end = 0;
+        pos = (uint32_t)(off & 12);
+        request();
+        top_up();
+        q = 0;
+        nb = 0;
+        peek();
+        fill();
+        drop(8 * (int)(off & 3));
+        peek();
+        fill();
+        peek();
     }
 };
 
-// One lane per segment (the format's unit of sequential decoding). Where rows and the column
-// side information are 16-byte aligned (row length a multiple of 8), a lane decodes its weights in
-// groups of 8: the group's cfi / scl read in one 16- and one 8-byte load, its 8 outputs written as
-// one 16-byte store; otherwise weight by weight.
-__global__ __launch_bounds__(256) void k_dec(const uint8_t* __restrict__ in, uint64_t in_blocks, const uint64_t* __restrict__ in_off,
-                                             uint8_t* __restrict__ dev, const TB* __restrict__ tb, const SG* __restrict__ sg,
-                                             int nseg, const int16_t* __restrict__ rfi, const int16_t* __restrict__ cfi,
-                                             const int8_t* __restrict__ scl, const int32_t* __restrict__ rowmap,
-                                             const uint8_t* __restrict__ dtab) {
-    const int s = (int)(xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x);
-    if (s >= nseg) return;
-    const SG g = sg[s];
+// A role's tables as the decoder holds them in LDS (113 KB; with the rings one workgroup per CU): for the 128 mantissa
+// contexts every symbol's cum | freq << 16 (129 words apart) and each bucket's first symbol; for the 512
+// exponent contexts the last 16 symbols' cumulative frequencies and the first of them; for the 16 sign
+// contexts the cumulative frequency of 1.
+constexpr int MC = 128, EC = 512, SC = 16, MSTRIDE = 129;
+struct DecTables {
+    uint4 exp[EC][2];
+    uint32_t man[MC * MSTRIDE];
+    uint32_t sgn[SC];
+    uint8_t first[MC][256];
+    uint8_t exp0[EC];
+};
+
+// One lane per segment (the format's unit of sequential decoding): bound by the latency of the chain
+// state -> table entry -> state, three symbols a weight. From the tables in global memory each link was an
+// L2 access (700 cycles a symbol). Here a role's tables are in LDS, and what is known before the state is
+// looked up ahead of it: the exponent's context is the prediction (the 16 likely symbols' bounds wait in
+// registers and are searched there) and the sign's its column's class; only the mantissa's context follows
+// from the symbol before it (two LDS reads). Rarer exponents, and tables with symbols no valid stream has,
+// go through the tables in global memory.
+// Lanes of one wave cost each other little, waves of one CU more, so a workgroup has as many waves as its
+// segments fill. Where they belong to more than one role, workgroup `part` of DEC_PARTS takes the part-th of
+// its run's roles (the last one the others too, one after another); a part without a role ends at once, and
+// the later parts come first in the grid, so that a run's roles are decoded side by side.
+// Measured, segments of 2^14 weights, ms before (tables in global memory, 64 segments to a workgroup) and
+// now: 40 segments 24.8 / 10.5, 640 31.8 / 11.3, 2560 32.1 / 12.0, 10240 32.3 / 10.7, 40960 32.4 / 12.3,
+// 163840 46.7 / 27.6 (640 ns a weight and lane with one wave to a CU).
+// Where rows and the column side information are 16-byte aligned (row length a multiple of 8), a lane
+// decodes its weights in groups of 8: the group's cfi / scl read in one 16- and one 8-byte load, its 8
+// outputs written as one 16-byte store; otherwise weight by weight.
+constexpr int DEC_T = 512, DEC_PARTS = 4;
+__global__ __launch_bounds__(DEC_T) void k_dec(const uint8_t* __restrict__ in, uint64_t in_blocks, const uint64_t* __restrict__ in_off,
+                                               uint8_t* __restrict__ dev, const TB* __restrict__ tb, const SG* __restrict__ sg,
+                                               int nseg, int per_wg, int nrun, const int16_t* __restrict__ rfi, const int16_t* __restrict__ cfi,
+                                               const int8_t* __restrict__ scl, const int32_t* __restrict__ rowmap,
+                                               const uint8_t* __restrict__ dtab) {
+    __shared__ __align__(16) DecTables L;
+    __shared__ __align__(16) uint4 ring[DEC_T][4];
+    __shared__ int role;
+    const int mine = (int)threadIdx.x, nt = (int)blockDim.x;
+    const int part = DEC_PARTS - 1 - (int)blockIdx.x / nrun;
+    const int64_t s = (int64_t)((int)blockIdx.x % nrun) * per_wg + mine;
+    bool todo = mine < per_wg && s < nseg;
+    const SG g = sg[todo ? s : 0];
     const TB T = tb[g.t];
-    uint16_t* W = reinterpret_cast<uint16_t*>(dev + T.doff);
-    Reader rd;
-    rd.start(in, in_off[s], in_blocks);
-    uint32_t x = 0;
-    for (int i = 0; i < 4; ++i) x = (x << 8) | rd.byte();
-    const uint8_t* dt = dtab + (size_t)T.tab * DT_BYTES;
-    const int16_t* cf = cfi + T.colbase;
-    const int8_t* sc = scl + T.colbase;
-    auto get = [&](int ctx) {
-        const uint32_t slot = x & (PSCALE - 1);
-        uint32_t c0, f;
-        const int v = dec_sym(dt + (size_t)ctx * DT_BYTES, slot, c0, f);
-        x = f * (x >> PB) + slot - c0;
-        // a valid stream needs at most two bytes here; the cap ends the loop on a damaged one
-#pragma unroll
-        for (int i = 0; i < 4 && x < RANS_L; ++i) x = (x << 8) | rd.byte();
-        return v;
-    };
-    auto weight = [&](int pred, int scv) {
-        const int ex = get(clampi(pred + 256, 0, 511));
-        const int man = get(512 + clampi(8 * ex - pred - 1016 + 64, 0, 127));
-        const int sgn = get(640 + scv);
-        return (uint32_t)((sgn << 15) | (ex << 7) | man);
-    };
-    Cursor cur;
-    cur.start(g.i0, T.rowlen);
-    int64_t orow = orig_row(T, rowmap, cur.rc);
-    int rf = rfi[T.rowbase + orow];
-    uint16_t* Wr = W + orow * T.rowlen;
-    const bool vec = (T.rowlen & 7) == 0 && (T.colbase & 7) == 0 && ((reinterpret_cast<uintptr_t>(W) & 15) == 0) &&
-                     ((reinterpret_cast<uintptr_t>(cfi) & 15) == 0) && ((reinterpret_cast<uintptr_t>(scl) & 7) == 0);
-    if (vec) {                                   // g.i0, g.n and the row length are multiples of 8
-        // the group's column side information (loaded one group ahead) and outputs move through
-        // 128-bit shift registers
-        uint4 c8n = *reinterpret_cast<const uint4*>(cf + cur.j);
-        uint2 s8n = *reinterpret_cast<const uint2*>(sc + cur.j);
-        for (int k = 0; k < g.n; k += 8) {
-            const int j = cur.j;
-            uint4 c8 = c8n;
-            uint64_t s64 = (uint64_t)s8n.x | ((uint64_t)s8n.y << 32);
-            const int jn = j + 8 < T.rowlen ? j + 8 : 0;
-            c8n = *reinterpret_cast<const uint4*>(cf + jn);
-            s8n = *reinterpret_cast<const uint2*>(sc + jn);
-            uint4 o = make_uint4(0u, 0u, 0u, 0u);
-            for (int t = 0; t < 8; ++t) {
-                const int cfv = (int)(int16_t)(uint16_t)c8.x;
-                c8.x = (c8.x >> 16) | (c8.y << 16);
-                c8.y = (c8.y >> 16) | (c8.z << 16);
-                c8.z = (c8.z >> 16) | (c8.w << 16);
-                c8.w >>= 16;
-                const int scv = (int)(int8_t)(uint8_t)s64;
-                s64 >>= 8;
-                const uint32_t v = weight(rf + cfv, scv);
-                o.x = (o.x >> 16) | (o.y << 16);
-                o.y = (o.y >> 16) | (o.z << 16);
-                o.z = (o.z >> 16) | (o.w << 16);
-                o.w = (o.w >> 16) | (v << 16);
+    for (int nth = 0;; ++nth) {
+        // the next role of the run; if it is this part's, its tables
+        __syncthreads();
+        if (threadIdx.x == 0) role = INT_MAX;
+        __syncthreads();
+        if (todo) atomicMin(&role, T.tab);
+        __syncthreads();
+        const int tab = role;
+        if (tab == INT_MAX || (nth > part && part < DEC_PARTS - 1)) return;
+        if (nth < part) {
+            if (T.tab == tab) todo = false;
+            continue;
+        }
+        const uint8_t* dt = dtab + (size_t)tab * DT_BYTES;
+        bool ok = true;
+        for (int i = mine; i < MC * 32; i += nt) {
+            const uint4 v = reinterpret_cast<const uint4*>(dt + (size_t)(EC + i / 32) * DT_BYTES + 2048)[i % 32];
+            uint32_t* o = L.man + (i / 32) * MSTRIDE + 4 * (i % 32);
+            o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
+        }
+        for (int i = mine; i < MC * 16; i += nt)
+            reinterpret_cast<uint4*>(L.first[i / 16])[i % 16] =
+                reinterpret_cast<const uint4*>(dt + (size_t)(EC + i / 16) * DT_BYTES + DT_FIRST)[i % 16];
+        for (int i = mine; i < MC; i += nt) {
+            L.man[i * MSTRIDE + 128] = PSCALE;
+            // cum[128] == 2^15: no symbol past 127
+            ok = ok && (reinterpret_cast<const uint32_t*>(dt + (size_t)(EC + i) * DT_BYTES + 2048)[128] & 0xffffu) == PSCALE;
+        }
+        for (int i = mine; i < EC; i += nt) {
+            const uint8_t* d = dt + (size_t)i * DT_BYTES + DT_LAST16;
+            L.exp[i][0] = reinterpret_cast<const uint4*>(d)[0];
+            L.exp[i][1] = reinterpret_cast<const uint4*>(d)[1];
+            L.exp0[i] = d[32];
+        }
+        if (threadIdx.x < SC) {
+            const uint32_t* ps = reinterpret_cast<const uint32_t*>(dt + (size_t)(EC + MC + threadIdx.x) * DT_BYTES + 2048);
+            L.sgn[threadIdx.x] = ps[1] & 0xffffu;
+            ok = ok && (ps[2] & 0xffffu) == PSCALE;
+        }
+        const bool in_lds = __syncthreads_and(ok) != 0;
+        if (!todo || T.tab != tab) continue;
+        todo = false;
+
+        uint16_t* W = reinterpret_cast<uint16_t*>(dev + T.doff);
+        Reader rd;
+        rd.start(in, in_off[s], in_blocks, ring[threadIdx.x]);
+        uint32_t x = (uint32_t)(rd.q >> 32);
+        rd.drop(32);
+        const int16_t* cf = cfi + T.colbase;
+        const int8_t* sc = scl + T.colbase;
+        // the state after a symbol of cumulative frequency c0 and frequency f: a valid stream needs at most two
+        // bytes here (x >= 2^8 before)
+        auto advance = [&](uint32_t slot, uint32_t c0, uint32_t f) __attribute__((always_inline)) {
+            x = f * (x >> PB) + slot - c0;
+            const int n = x >= RANS_L ? 0 : (x >= RANS_L >> 8 ? 8 : 16);
+            x = (uint32_t)(((((uint64_t)x << 32) | (uint32_t)(rd.q >> 32)) << n) >> 32);
+            rd.drop(n);
+        };
+        auto from_global = [&](int ctx) __attribute__((always_inline)) {
+            uint32_t c0, f;
+            const uint32_t slot = x & (PSCALE - 1);
+            const int v = dec_sym(dt + (size_t)ctx * DT_BYTES, slot, c0, f);
+            advance(slot, c0, f);
+            return v;
+        };
+        // a weight whose exponent's bounds (a, b) and first symbol e0 are at hand
+        auto weight = [&](int pred, int scv, uint4 a, uint4 b, int e0) __attribute__((always_inline)) {
+            if (rd.nb <= 32) rd.fill();
+            const bool plain_sign = (uint32_t)scv < (uint32_t)SC;
+            const uint32_t one = L.sgn[scv & (SC - 1)];
+            // exponent: the last of the 16 bounds at or below the slot, by halves
+            int ex;
+            uint32_t slot = x & (PSCALE - 1);
+            if (in_lds && slot >= (a.x & 0xffffu)) {
+                uint32_t up = PSCALE, piv = b.x & 0xffffu;
+                bool hi = slot >= piv;
+                uint4 h = hi ? b : a;
+                ex = hi ? 8 : 0;
+                up = hi ? up : piv;
+                piv = h.z & 0xffffu;
+                hi = slot >= piv;
+                uint32_t h0 = hi ? h.z : h.x, h1 = hi ? h.w : h.y;
+                ex += hi ? 4 : 0;
+                up = hi ? up : piv;
+                piv = h1 & 0xffffu;
+                hi = slot >= piv;
+                h0 = hi ? h1 : h0;
+                ex += hi ? 2 : 0;
+                up = hi ? up : piv;
+                piv = h0 >> 16;
+                hi = slot >= piv;
+                const uint32_t c0 = hi ? piv : h0 & 0xffffu;
+                ex += hi ? 1 : 0;
+                up = hi ? up : piv;
+                ex += e0;
+                advance(slot, c0, up - c0);
+            } else {
+                ex = from_global(clampi(pred + 256, 0, 511));
             }
-            *reinterpret_cast<uint4*>(Wr + j) = o;
-            cur.j += 8;
-            if (cur.j == T.rowlen && k + 8 < g.n) {
+            // mantissa: the slot's bucket names its first symbol, one of the next holds the slot
+            const int mc = clampi(8 * ex - pred - 1016 + 64, 0, 127);
+            int man;
+            if (in_lds) {
+                slot = x & (PSCALE - 1);
+                const uint32_t* m = L.man + mc * MSTRIDE;
+                man = L.first[mc][slot >> 7];
+                uint32_t u = m[man], v = m[man + 1];
+                while (slot >= (u & 0xffffu) + (u >> 16)) {
+                    u = v;
+                    ++man;
+                    v = m[man + 1 < MC ? man + 1 : MC];
+                }
+                advance(slot, u & 0xffffu, u >> 16);
+            } else {
+                man = from_global(512 + mc);
+            }
+            if (rd.nb < 16) {                        // rare: the two symbols took 17 bits or more
+                rd.peek();
+                rd.fill();
+            }
+            int sign;
+            if (in_lds && plain_sign) {
+                slot = x & (PSCALE - 1);
+                sign = slot >= one ? 1 : 0;
+                advance(slot, sign ? one : 0u, sign ? PSCALE - one : one);
+            } else {
+                sign = from_global(640 + scv);
+            }
+            rd.peek();
+            return (uint32_t)((sign << 15) | (ex << 7) | man);
+        };
+        Cursor cur;
+        cur.start(g.i0, T.rowlen);
+        int64_t orow = orig_row(T, rowmap, cur.rc);
+        int rf = rfi[T.rowbase + orow];
+        uint16_t* Wr = W + orow * T.rowlen;
+        const bool vec = (T.rowlen & 7) == 0 && (T.colbase & 7) == 0 && ((reinterpret_cast<uintptr_t>(W) & 15) == 0) &&
+                         ((reinterpret_cast<uintptr_t>(cfi) & 15) == 0) && ((reinterpret_cast<uintptr_t>(scl) & 7) == 0);
+        if (vec) {                                   // g.i0, g.n and the row length are multiples of 8
+            // the group's column side information (loaded one group ahead) and outputs move through
+            // 128-bit shift registers
+            uint4 c8n = *reinterpret_cast<const uint4*>(cf + cur.j);
+            uint2 s8n = *reinterpret_cast<const uint2*>(sc + cur.j);
+            for (int k = 0; k < g.n; k += 8) {
+                const int j = cur.j;
+                uint4 c8 = c8n;
+                uint64_t s64 = (uint64_t)s8n.x | ((uint64_t)s8n.y << 32);
+                const int jn = j + 8 < T.rowlen ? j + 8 : 0;
+                c8n = *reinterpret_cast<const uint4*>(cf + jn);
+                s8n = *reinterpret_cast<const uint2*>(sc + jn);
+                uint4 o = make_uint4(0u, 0u, 0u, 0u);
+                int pred = rf + (int)(int16_t)(uint16_t)c8.x;
+                int pe = clampi(pred + 256, 0, 511);
+                uint4 a = L.exp[pe][0], b = L.exp[pe][1];
+                int e0 = L.exp0[pe];
+                for (int t = 0; t < 8; ++t) {
+                    if (t % 4 == 0) rd.top_up();
+                    c8.x = (c8.x >> 16) | (c8.y << 16);
+                    c8.y = (c8.y >> 16) | (c8.z << 16);
+                    c8.z = (c8.z >> 16) | (c8.w << 16);
+                    c8.w >>= 16;
+                    const int scv = (int)(int8_t)(uint8_t)s64;
+                    s64 >>= 8;
+                    // the next weight's bounds, on their way while this one is decoded
+                    const int pred1 = rf + (int)(int16_t)(uint16_t)c8.x;
+                    pe = clampi(pred1 + 256, 0, 511);
+                    const uint4 a1 = L.exp[pe][0], b1 = L.exp[pe][1];
+                    const int e1 = L.exp0[pe];
+                    const uint32_t v = weight(pred, scv, a, b, e0);
+                    o.x = (o.x >> 16) | (o.y << 16);
+                    o.y = (o.y >> 16) | (o.z << 16);
+                    o.z = (o.z >> 16) | (o.w << 16);
+                    o.w = (o.w >> 16) | (v << 16);
+                    pred = pred1;
+                    a = a1;
+                    b = b1;
+                    e0 = e1;
+                }
+                *reinterpret_cast<uint4*>(Wr + j) = o;
+                cur.j += 8;
+                if (cur.j == T.rowlen && k + 8 < g.n) {
+                    cur.j = 0;
+                    ++cur.rc;
+                    orow = orig_row(T, rowmap, cur.rc);
+                    rf = rfi[T.rowbase + orow];
+                    Wr = W + orow * T.rowlen;
+                }
+            }
+            continue;
+        }
+        for (int k = 0; k < g.n; ++k) {
+            const int j = cur.j, pred = rf + cf[j], pe = clampi(pred + 256, 0, 511);
+            if (k % 4 == 0) rd.top_up();
+            Wr[j] = (uint16_t)weight(pred, sc[j], L.exp[pe][0], L.exp[pe][1], L.exp0[pe]);
+            if (++cur.j == T.rowlen && k + 1 < g.n) {
                 cur.j = 0;
                 ++cur.rc;
                 orow = orig_row(T, rowmap, cur.rc);
                 rf = rfi[T.rowbase + orow];
                 Wr = W + orow * T.rowlen;
             }
-        }
-        return;
-    }
-    for (int k = 0; k < g.n; ++k) {
-        const int j = cur.j;
-        Wr[j] = (uint16_t)weight(rf + cf[j], sc[j]);
-        if (++cur.j == T.rowlen && k + 1 < g.n) {
-            cur.j = 0;
-            ++cur.rc;
-            orow = orig_row(T, rowmap, cur.rc);
-            rf = rfi[T.rowbase + orow];
-            Wr = W + orow * T.rowlen;
         }
     }
 }
@@ -746,9 +926,15 @@ int spa_r2_decode(const void* in, uint64_t in_bytes, const uint64_t* in_off, voi
     if (nseg < 0) return fail(SPA_ERR_ARG, "spa_r2_decode: negative segment count");
     if (nseg == 0) return SPA_OK;
     if (reinterpret_cast<uintptr_t>(in) & 15) return fail(SPA_ERR_ARG, "spa_r2_decode: stream not 16-byte aligned");
-    hipLaunchKernelGGL(k_dec, dim3((unsigned)((nseg + 255) / 256)), dim3(256), 0, (hipStream_t)stream, (const uint8_t*)in,
-                       (in_bytes + 15) / 16, in_off, (uint8_t*)dev, (const TB*)tb, (const SG*)sg, nseg, rfi, cfi, scl, rowmap,
-                       dtab);
+    // A workgroup's tables fill a CU's LDS. Up to 200 workgroups run side by side (2560 segments took 12.0 ms
+    // on 100 to 230, 19.9 ms on 240 and 21.4 ms on 256, where some CUs are given two while others idle); more
+    // segments than those hold go in rounds of them.
+    constexpr int SIDE = 200;
+    const int rounds = (nseg + SIDE * DEC_T - 1) / (SIDE * DEC_T);
+    const int per_wg = (nseg + SIDE * rounds - 1) / (SIDE * rounds), nrun = (nseg + per_wg - 1) / per_wg;
+    hipLaunchKernelGGL(k_dec, dim3((unsigned)(nrun * DEC_PARTS)), dim3((unsigned)((per_wg + 63) / 64 * 64)), 0, (hipStream_t)stream,
+                       (const uint8_t*)in, (in_bytes + 15) / 16, in_off, (uint8_t*)dev, (const TB*)tb, (const SG*)sg, nseg, per_wg,
+                       nrun, rfi, cfi, scl, rowmap, dtab);
     SPA_HIP_TRY(hipGetLastError());
     return SPA_OK;
 }

@@ -272,3 +272,30 @@ def test_hip_r2_grouped_equals_one_pass(name):
     host = np.frombuffer(data, np.uint8)
     for off, nb, _, _ in layout["t"]:
         assert out[off:off + nb].tobytes() == host[off:off + nb].tobytes()
+
+
+@pytest.mark.parametrize("spread", [0, 30])
+def test_hip_r2_decode_workgroups_of_several_roles(spread):
+    """a run of six segments per workgroup that holds one role, several, or more roles than there are parts
+    of its workgroups; row lengths that are read in groups of eight and that are not; exponents within the
+    16 likely symbols of their contexts and, spread over 60 octaves, far outside them"""
+    say("case r2 several roles", spread)
+    g = np.random.Generator(np.random.PCG64(51))
+    shapes = [(1 + i % 2, (999, 1024, 8, 4097, 17)[i % 5]) for i in range(13)]
+    shapes[6] = (1150, r2.SEG)
+    data, ts = b"", []
+    for i, (n, rl) in enumerate(shapes):
+        x = g.normal(0, 0.02, (n, rl))
+        if spread:
+            x *= np.exp2(np.rint(g.uniform(-spread, spread, (n, rl))))
+        w = synth.bf16_bits(x.astype(np.float32))
+        ts.append((f"blk.0.role{i}.weight", len(data), w.nbytes, rl))
+        data += w.tobytes()
+    layout = r2.layout_of(ts, len(data))
+    codec = r2.BF16v2(group_bytes=1 << 30)
+    parts = codec.compress(data, layout)
+    assert len(parts["arrays"]["lens"]) > 1150
+    out = codec.decompress(parts)
+    host = np.frombuffer(data, np.uint8)
+    for off, nb, _, _ in layout["t"]:
+        assert out[off:off + nb].tobytes() == host[off:off + nb].tobytes()
