@@ -481,9 +481,34 @@ __device__ __forceinline__ void seed_val(int st, const uint8_t* sb, int64_t gw, 
     else seed_val_any(st, sb, gw, cols, x, h);
 }
 
+// eight weights' seed values, the first a multiple of 8: a BF16 seed's 16 bytes in one load where they are
+// aligned (a load and a wait a byte pair otherwise, one weight after another)
+__device__ __forceinline__ void seed_vals8(int st, const uint8_t* sb, int64_t gw, int cols, float (&x)[8], float (&h)[8]) {
+    const uint8_t* p = sb + 2 * gw;
+    if (st == 30 && (reinterpret_cast<uintptr_t>(p) & 15) == 0) {
+        const uint4 v = *reinterpret_cast<const uint4*>(p);
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            x[t] = __uint_as_float(t & 1 ? w[t / 2] & 0xffff0000u : w[t / 2] << 16);
+            h[t] = 0.f;
+        }
+        return;
+    }
+#pragma unroll
+    for (int t = 0; t < 8; ++t) seed_val(st, sb, gw + t, cols, x[t], h[t]);
+}
+
 // position of a weight's column in its row: the first 256 columns, then 7 parts
 __device__ __forceinline__ int pos8(int64_t col, int cols) {
-    return cols <= 0 || col < 256 ? 0 : 1 + (int)min((int64_t)6, col * 7 / cols);
+    if (cols <= 0 || col < 256) return 0;
+    // col * 7 / cols as the count of the parts' starts at or below it: six compares, where the 64-bit
+    // division is some hundred instructions a weight
+    const uint64_t c7 = (uint64_t)col * 7;
+    int n = 1;
+#pragma unroll
+    for (int k = 1; k <= 6; ++k) n += c7 >= (uint64_t)(uint32_t)cols * k ? 1 : 0;
+    return n;
 }
 
 __device__ __forceinline__ int hboff_of(const TM& m) { return m.seed_type == SEED_COLRMS ? HBOFF_COL : HBOFF; }

@@ -159,3 +159,25 @@ def test_hip_lut32_folds_freq_and_cum_into_the_symbol_table():
         assert np.array_equal(sym, a[t]), t
         assert np.array_equal(((e[t] >> 8) & 4095) + 1, freq[t][sym]), t
         assert np.array_equal(e[t] >> 20, slots - cum[t][sym]), t
+
+
+@pytest.mark.parametrize("shift", [0, 2, 16])
+@pytest.mark.parametrize("name", ["q4_k", "q8_0"])
+def test_hip_qr_decode_seed_alignment(vectors, name, shift):
+    """a seed that starts on a multiple of 16 bytes (read eight weights at a time) and one that does not"""
+    name = next(c[0] for c in CASES if c[0].lower().startswith(name))
+    T, cols, F, P, seed = case_inputs(vectors, name)
+    say("case qr decode seed alignment", name, shift)
+    sd = dev.DeviceArray.from_host(np.concatenate([np.zeros(shift, np.uint8), seed.view(np.uint8).reshape(-1)]))
+    out = qr.decode_parts(T, vectors[f"{name}/freq"], vectors[f"{name}/used"], vectors[f"{name}/lens"],
+                          vectors[f"{name}/stream"].tobytes(), [(P, shift, 30, cols, -1)], sd)
+    assert np.array_equal(out.to_host()[:len(F)], F)
+
+
+def test_column_parts_equal_the_division():
+    """the count of the parts' starts at or below a column against the definition min(6, 7 col / cols)"""
+    for cols in (257, 512, 1000, 4096, 16384, 2**31 - 1):
+        col = np.unique(np.clip(np.concatenate([np.arange(256, 20000), [k * cols // 7 + d for k in range(1, 8) for d in (-1, 0, 1)]]), 256, cols + 255))
+        c7 = 7 * col.astype(np.int64)
+        n = sum((c7 >= cols * k).astype(np.int64) for k in range(1, 7))
+        assert np.array_equal(n, np.minimum(6, c7 // cols)), cols
