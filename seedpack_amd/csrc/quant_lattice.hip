@@ -17,16 +17,23 @@
 // q and q^2 give both.
 // Exactness: the filter's answer counts only where its best point leads the second by more than a bound
 // on everything that separates it from the reference's float sums (tolerance() below). Otherwise, and
-// for inputs outside the filter's range, the wave evaluates the reference's float expression for the
-// whole list (exact_neighbour), its first strict minimum winning as in the C code.
+// for inputs outside the filter's range, the reference's float expression is evaluated for the whole list,
+// its first strict minimum winning as in the C code: a few lanes' lists one after another, each by the whole
+// wave (exact_neighbour), more of them cut into pieces that are dealt to the lanes (dealt_neighbours).
 //
 // Bound by VALU issue. With the importance matrix, against one list search per trial and group: IQ2_XS
 // 4096 x 12288 6.10 to 3.14 ms (7231 to about 2450 lane-instructions a weight), IQ3_XXS 2053 x 3584 1.157
 // to 0.638 ms; on 4096 x 4096 IQ2_XXS 1.38 to 0.92 ms, IQ2_S 0.68 to 0.50 ms, IQ3_S 1.24 to 0.76 ms.
+// Weights on a coarse grid, where equal distances are common, need the float sums for up to half of their trials.
+// Without the importance matrix, 4096 x 4096, us: one list search per trial and group; undecided lists one after
+// another, each by the whole wave; dealt, up to four trials at once:
+//   4-bit codes, a scale per 32    IQ2_S 712 / 3790 / 945    IQ3_XXS 1835 / 5220 / 1790    IQ3_S 1290 / 3150 / 1290
+//   three values, a scale per 128  IQ2_S 556 / 2600 / 584    IQ3_XXS 1600 / 15460 / 1490   IQ3_S  885 / 2960 /  785
+// On normal weights the dealt search, which runs there now and then, and its registers cost 1% to 2%, IQ2_S 4%.
 //
 // Mapping: one lane per sub-block (32 or 16 weights), G = 256/N lanes per super-block, 256-lane
-// workgroups, held to three waves per SIMD (a few registers spill; at two or four waves the kernels are
-// 10-20% slower). The groups of the sub-blocks are worked through one by one, a group's weights read again
+// workgroups, held to three waves per SIMD (8 to 212 bytes of scratch a lane; at two or four waves the kernels
+// are 10-20% slower). The groups of the sub-blocks are worked through one by one, a group's weights read again
 // for each (they stay in L1/L2) so that only the trials' running sums are held in registers.
 #include "../../include/seedpack_amd.h"
 #include "common.h"
@@ -40,8 +47,14 @@ namespace {
 constexpr int WG = 256;
 constexpr float FLT_BIG = 3.402823466e+38F;   // FLT_MAX
 constexpr uint32_t PREV = 0xffffu;            // a trial's point: that of the trial before it
-constexpr uint32_t EXACT = 0xfffeu;           // a trial's point: still to be found by exact_neighbour
+constexpr uint32_t EXACT = 0xfffeu;           // a trial's point: still to be found by the float sums
+// Open points of at most FEW lanes and FEW_TRIALS trials are found one after another, more of them dealt. (FEW = 0,
+// 2, 6: IQ2_S with normal weights 631, 606, 606 us; 6 is 10-25% slower where weights are on a fine grid.) A run that
+// is undecided at both ends is left open at once where more than MANY runs searched side by side are undecided;
+// elsewhere a near miss of one or two trials is likelier, which a further scan of the run costs less.
+constexpr int FEW = 2, FEW_TRIALS = 4, MANY = 6;
 constexpr int QCAP = 256;                     // runs a wave queues before it searches them
+constexpr uint32_t PEELED = 1u << 31;         // a queued run: what is left of one with an undecided end
 
 enum Kind { K_IQ2_XXS, K_IQ2_XS, K_IQ2_S, K_IQ3_XXS, K_IQ3_S };
 
@@ -227,6 +240,84 @@ __device__ __forceinline__ int exact_neighbour(const float (&xval)[D], const flo
     return bj;
 }
 
+// The same for every lane with bits in `sel`, each its own group and list, at NT scales at once: trials t0 to
+// t0 + NT - 1, bit i for trial t0 + i (NT = 1: the scale s). The lists are cut into pieces of R entries and dealt to
+// the lanes in rounds, so that the wave does not wait for its longest list. A list's winner is the least of d2 as
+// bits, position and point (d2 is not negative; infinities and NaN order above FLT_MAX), lowered by atomic minima
+// in the words of the queue, which is empty here.
+template <int K, int NT>
+__device__ __forceinline__ void dealt_neighbours(WaveMem<K>& W, int t0, uint32_t sel, const float (&xval)[Cfg<K>::D],
+                                                 const float (&v)[Cfg<K>::D], float max, float s, int gi,
+                                                 const Point<Cfg<K>::D>* pts, const uint16_t* __restrict__ nb) {
+    constexpr int D = Cfg<K>::D, R = Cfg<K>::R;
+    static_assert(64 * NT <= QCAP, "a word for each lane and scale");
+    unsigned long long* slots = reinterpret_cast<unsigned long long*>(W.queue);
+    const int lane = (int)__lane_id();
+    const int np = sel ? (list_length(gi) + R - 1) / R : 0;
+    const unsigned long long none = ((unsigned long long)0x7f7fffffu << 32) | (sel ? nb[list_offset(gi)] : 0u);   // (FLT_MAX, position 0)
+#pragma unroll
+    for (int i = 0; i < NT; ++i) slots[64 * i + lane] = none;
+    // inclusive prefix of the piece counts: shifts by 1, 2, 4, 8 within a row of 16 lanes, then the rows below
+    int incl = np;
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x111, 0xf, 0xf, false);
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x112, 0xf, 0xf, false);
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x114, 0xf, 0xf, false);
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x118, 0xf, 0xf, false);
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x142, 0xa, 0xf, false);
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x143, 0xc, 0xf, false);
+    const int total = __builtin_amdgcn_readlane(incl, 63);
+    wave_lds_sync();
+    for (int base = 0; base < total; base += 64) {
+        const int q = base + lane;
+        int o = 0;                               // the lane whose pieces hold q: how many end at or before it
+#pragma unroll
+        for (int st = 32; st >= 1; st >>= 1)
+            if (__shfl(incl, o + st - 1) <= q) o += st;
+        const int first = __shfl(incl - np, o), g = __shfl(gi, o);
+        uint32_t what = (uint32_t)__shfl((int)(sel | (uint32_t)t0 << 8), o);         // by all lanes, before any is left out
+        if (q >= total) what = 0u;
+        const float m = __shfl(NT == 1 ? s : max, o);
+        float x[D], w[D];
+#pragma unroll
+        for (int i = 0; i < D; ++i) { x[i] = __shfl(xval[i], o); w[i] = __shfl(v[i], o); }
+        const int p = q - first, len = list_length(g);
+        const uint16_t* list = what ? nb + list_offset(g) + p * R : nb;      // (lists are padded to whole pieces)
+        float sc[NT];
+        unsigned long long best[NT];
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            sc[i] = NT == 1 ? m : 1 / (trial_num<K>((int)(what >> 8) + i) / m);
+            best[i] = ~0ull;
+        }
+#pragma unroll 1
+        for (int e = 0; e < R; ++e) {
+            const int j = list[e];
+            const uint32_t low = (uint32_t)((p * R + e) << 16) | (uint32_t)j;
+            float c[D];
+            coords<D>(pts[j], c);
+#pragma unroll
+            for (int i = 0; i < NT; ++i) {
+                float d2 = 0;
+#pragma unroll
+                for (int b = 0; b < D; ++b) {
+                    const float diff = sc[i] * c[b] - x[b];
+                    d2 += w[b] * diff * diff;
+                }
+                const unsigned long long key = ((unsigned long long)__float_as_uint(d2) << 32) | low;
+                if (p * R + e < len && key < best[i]) best[i] = key;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+            if (what >> i & 1) atomicMin(&slots[64 * i + o], best[i]);
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+        if (sel >> i & 1) W.point[t0 + i][lane] = (uint16_t)slots[64 * i + lane];
+    wave_lds_sync();
+}
+
 // ---------------------------------------------------------------- the filter
 
 // Bounds over every list of a lattice type (tests/test_iq_tables.py checks them against the tables):
@@ -337,8 +428,8 @@ __device__ __forceinline__ void sums(const uint32_t (&w)[D == 8 ? 12 : 8], const
 //     better of the two all the way: the trials before the crossing take g, the others h. If it does not, the
 //     two trials at the crossing are searched as well (the run queued again with them): g and h there mean
 //     the same; anything else leaves a shorter run on one side to be searched the same way.
-// A queue entry: {map entry, lane | first trial << 8 | last << 16 | (trial before the crossing + 1) << 24}.
-// Returns the trials (as bits) of which some point is left to exact_neighbour.
+// A queue entry: {map entry, lane | first trial << 8 | last << 16 | (trial before the crossing + 1) << 24 | PEELED}.
+// Returns the trials (as bits) of which some point is left open (EXACT).
 template <int K, bool FINAL>
 __device__ __forceinline__ uint32_t search_runs(WaveMem<K>& W, int count, const Point<Cfg<K>::D>* pts, const uint16_t* __restrict__ nb) {
     constexpr int D = Cfg<K>::D, NS = FINAL ? 1 : 2, R = Cfg<K>::R;
@@ -352,8 +443,8 @@ __device__ __forceinline__ uint32_t search_runs(WaveMem<K>& W, int count, const 
         const bool act = (lane >> share) < n;
         const uint2 task = W.queue[(head + (act ? lane >> share : 0)) & (QCAP - 1)];
         const int o = (int)(task.y & 63u), r0 = (int)((task.y >> 8) & 31u), r1 = (int)((task.y >> 16) & 31u);
-        const bool inner = task.y >> 24 != 0;             // the two trials at a crossing inside r0 .. r1
-        const int t0 = inner ? (int)(task.y >> 24) - 1 : r0, t1 = inner ? t0 + 1 : r1;
+        const bool inner = (task.y >> 24 & 63u) != 0;     // the two trials at a crossing inside r0 .. r1
+        const int t0 = inner ? (int)(task.y >> 24 & 63u) - 1 : r0, t1 = inner ? t0 + 1 : r1;
         const int gi = (int)task.x, np = act ? (list_length(gi) + R - 1) / R : 0;
         const uint16_t* list = nb + list_offset(gi);
         const Piece<R>* pieces = reinterpret_cast<const Piece<R>*>(list);
@@ -431,7 +522,14 @@ __device__ __forceinline__ uint32_t search_runs(WaveMem<K>& W, int count, const 
             sure[k] = m2[k] - m1[k] > tol && id[k] < Cfg<K>::PTS;
             all = all && sure[k];
         }
+        auto leave_open = [&](int from, int to) __attribute__((always_inline)) {
+            for (int t = from; t <= to; ++t) {
+                W.point[t][o] = (uint16_t)EXACT;
+                open |= 1u << t;
+            }
+        };
         uint32_t again = 0, more = 0;      // runs to queue again
+        const bool many = __popcll(__ballot(act && part == 0 && !all)) > MANY;
         if (act && part == 0) {
             if (!sure[0]) open |= 1u << (FINAL ? 0 : t0);
             if (!sure[NS - 1]) open |= 1u << (FINAL ? 0 : t1);
@@ -458,8 +556,11 @@ __device__ __forceinline__ uint32_t search_runs(WaveMem<K>& W, int count, const 
                             W.point[tx][o] = (uint16_t)h;
                         else
                             again = (task.y & 0xffffffu) | ((uint32_t)tx << 24);
+                    } else if (task.y & PEELED || (many && !sure[0] && !sure[NS - 1])) {
+                        // undecided once more, or at both ends in many lanes: equal distances, which last
+                        leave_open(t0, t1);
                     } else {
-                        again = (uint32_t)o | ((uint32_t)(t0 + 1) << 8) | ((uint32_t)(t1 - 1) << 16);
+                        again = (uint32_t)o | ((uint32_t)(t0 + 1) << 8) | ((uint32_t)(t1 - 1) << 16) | PEELED;
                     }
                 }
             } else {
@@ -482,10 +583,7 @@ __device__ __forceinline__ uint32_t search_runs(WaveMem<K>& W, int count, const 
                 if (room) {
                     W.queue[(tail + lanes_below(m)) & (QCAP - 1)] = make_uint2(task.x, more);
                 } else {
-                    for (int t = t1 + 1; t < r1; ++t) {
-                        W.point[t][o] = (uint16_t)EXACT;
-                        open |= 1u << t;
-                    }
+                    leave_open(t1 + 1, r1 - 1);
                 }
             }
             tail += room ? __popcll(m) : 0;
@@ -685,11 +783,16 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(3))) void k_
         return any_odd ? round_exact<D, KMAXQ>(xval, id) : round_float<D, KMAXQ>(xval, id);
     };
     auto id_at = [&](int t, float m, float rm) { return any_odd ? trial_num<K>(t) / m : trial_id<K>(t, m, rm); };
-    // the points still open (EXACT) of trial t at scale s, found by the wave one lane at a time
-    auto settle = [&](int t, const float (&xval)[D], const float (&v)[D], float s, int u) __attribute__((always_inline)) {
-        uint64_t m = __ballot(W.point[t][lane] == EXACT);
+    // the points still open (EXACT) of trial t at scale s
+    auto settle = [&](bool last, int t, const float (&xval)[D], const float (&v)[D], float s, int u) __attribute__((always_inline)) {
+        const bool off = W.point[t][lane] == EXACT;
+        uint64_t m = __ballot(off);
         if (!m) return;
         const int gi = tab.map[u];
+        if (last && __popcll(m) > FEW) {
+            dealt_neighbours<K, 1>(W, 0, off ? 1u : 0u, xval, v, max, s, gi, pts, tab.nb);
+            return;
+        }
         for (; m; m &= m - 1) {
             const int o = __ffsll((unsigned long long)m) - 1;
             const int j = exact_neighbour<D>(xval, v, s, gi, o, pts, tab.nb);
@@ -718,8 +821,9 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(3))) void k_
             }
         }
         uint32_t open = any_by_hand ? ~0u >> (32 - T) : 0u;
+        const uint32_t starts = filter ? level_changes<K>(xval, max, rmax) : ~0u;      // of runs of one rounding
         int n = 0;
-        for (uint32_t left = filter ? level_changes<K>(xval, max, rmax) : 0u; __ballot(left != 0); ) {
+        for (uint32_t left = filter ? starts : 0u; __ballot(left != 0); ) {
             const int from = __ffs((int)left) - 1, to = (left & (left - 1)) ? __ffs((int)(left & (left - 1))) - 2 : T - 1;
             const int u = round_float<D, KMAXQ>(xval, trial_id<K>(from, max, rmax));
             const uint64_t m = __ballot(left != 0);
@@ -733,10 +837,27 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(3))) void k_
                 n = 0;
             }
         }
-        for (; open; open &= open - 1) {
-            const int t = __ffs((int)open) - 1;
-            const float id = id_at(t, max, rmax);
-            settle(t, xval, v, 1 / id, round_at(xval, id));
+        uint32_t mine = 0;
+        for (uint32_t m = open; m; m &= m - 1) {
+            const int t = __ffs((int)m) - 1;
+            mine |= W.point[t][lane] == EXACT ? 1u << t : 0u;
+        }
+        if (__popcll(__ballot(mine != 0)) > FEW || __popc(open) > FEW_TRIALS) {
+            // up to four trials of a run at once
+            while (__ballot(mine != 0)) {
+                const int t = mine ? __ffs((int)mine) - 1 : 0;
+                const uint32_t later = starts & ~1u << t, run = later ? (later & (0u - later)) - 1 : ~0u;     // before the next run
+                const uint32_t now = mine & run & 15u << t;
+                const int gi = tab.map[round_at(xval, id_at(t, max, rmax))];
+                dealt_neighbours<K, 4>(W, t, now >> t, xval, v, max, 0.f, gi, pts, tab.nb);
+                mine &= ~now;
+            }
+        } else {
+            for (; open; open &= open - 1) {
+                const int t = __ffs((int)open) - 1;
+                const float id = id_at(t, max, rmax);
+                settle(false, t, xval, v, 1 / id, round_at(xval, id));
+            }
         }
         float wx[D];
 #pragma unroll
@@ -800,7 +921,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(3))) void k_
         wave_lds_sync();
         const int n = sort_runs<K>(W, __popcll(m), tab.map);
         search_runs<K, true>(W, n, pts, tab.nb);
-        settle(0, xval, v, redo ? scale : 1 / bid, u);
+        settle(true, 0, xval, v, redo ? scale : 1 / bid, u);
         const int p = W.point[0][lane];
         W.best[k][lane] = (uint16_t)p;
         float q[D];
