@@ -143,6 +143,13 @@ int spa_dequantize(int ggml_type, const void* src, int64_t nrows, int64_t n_per_
 int spa_iq_table_host(int index, const void** grid, int* grid_bytes, const int32_t** map, int* map_n,
                       const uint16_t** neighbours, int* nb_n);
 
+/* What the exactness of the lattice types' searches rests on (16, 17, 18, 21, 22), by the code the kernels run:
+ * the inverse scale of a trial for n sub-block maxima, and the bound on a lead for {scale, 1 / scale, A, C, B, best
+ * value} in the searches' units, followed by the spreads of the neighbour lists that it assumes (first point to
+ * another: q, q^2; any two points: q, q^2). Host memory, no device call. */
+int spa_lattice_trials_host(int ggml_type, int trial, const float* max, int64_t n, float* id);
+int spa_lattice_bound_host(int ggml_type, const float* terms, float* out5);
+
 /* ---- QR residual coder (all 20 quant types; seedpack/qr.py) ----
  * Batch descriptors are device arrays with the reference's byte layout (qr.py:898-900):
  *   tm: one 32-byte record per tensor {i64 blk0, i64 seed_off, i32 seed_type, i32 cols, i64 imx_off}

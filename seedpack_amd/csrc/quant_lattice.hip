@@ -35,6 +35,8 @@
 // workgroups, held to three waves per SIMD (8 to 212 bytes of scratch a lane; at two or four waves the kernels
 // are 10-20% slower). The groups of the sub-blocks are worked through one by one, a group's weights read again
 // for each (they stay in L1/L2) so that only the trials' running sums are held in registers.
+#include <type_traits>
+
 #include "../../include/seedpack_amd.h"
 #include "common.h"
 #include "iq_tables.h"
@@ -160,14 +162,14 @@ __device__ __forceinline__ int round_float(const float (&xval)[D], float id) {
 }
 
 template <int K>
-__device__ __forceinline__ float trial_num(int t) {
+__host__ __device__ __forceinline__ float trial_num(int t) {
     return (float)(2 * Cfg<K>::KMAXQ - 1) + (float)(t + Cfg<K>::IS_LO) * Cfg<K>::STEP;
 }
 // trial t's inverse scale num / max, correctly rounded: with rmax = 1 / max correctly rounded, one
 // remainder step corrects num rmax to the quotient (checked for every mantissa of max and every num of
 // the types; max is within 2^+-60 here, so nothing over- or underflows)
 template <int K>
-__device__ __forceinline__ float trial_id(int t, float max, float rmax) {
+__host__ __device__ __forceinline__ float trial_id(int t, float max, float rmax) {
     const float num = trial_num<K>(t), q = num * rmax;
     return __builtin_fmaf(__builtin_fmaf(-max, q, num), rmax, q);
 }
@@ -320,7 +322,7 @@ __device__ __forceinline__ void dealt_neighbours(WaveMem<K>& W, int t0, uint32_t
 
 // ---------------------------------------------------------------- the filter
 
-// Bounds over every list of a lattice type (tests/test_iq_tables.py checks them against the tables):
+// Bounds over every list of a lattice type (spa_lattice_bound_host shows them to the tests):
 // L1, M2: the largest sums over the coordinates of |q - q'| and |q^2 - q'^2| between a list's first
 // point and another of it; P1, P2: between any two points of it.
 template <int D> struct ListBound;
@@ -329,18 +331,22 @@ template <> struct ListBound<4> { static constexpr float L1 = 16, M2 = 336, P1 =
 
 // How far the filter's second best value has to lie above its best so that the best is the reference's
 // strict minimum. The values are F = s' C - B over integers, s' = s 2^b / 2^(a+1), relative to the list's
-// first point; d2 = A + 2 s / 2^b F. With u = 2^-24, |V| <= 2^23 and |P| < 2^23 it covers, for two points:
-//   rounding V = v 2^a to an integer    s' P2 / 2          rounding P = v x 2^b (and v x)    P1 (0.5 + 0.5)
-//   s' (2 u relative)                   s' P2              converting C, B and the fma       2 (s' M2 + L1 / 2)
-//   the reference's float sum: 12 u d2 + u s^2 C for each point (products of rounded differences added left
-//   to right; 2 |diff| s q <= diff^2 + s^2 q^2)            24 u d2 2^b / (2 s) + 2 u s' C
-// with the whole enlarged by a quarter. d2 in these units is A 2^b / (2 s) + F.
+// first point; d2 = A + 2 s / 2^b F. With u = 2^-24, V = v 2^a <= VMAX = 2^23 (2^22 for D = 4) and
+// |P| = |v x 2^b| < 2^23 it covers, for the two points:
+//   V rounded to an integer      s' P2 / 2          P rounded to an integer, and v x itself     P1 / 2 + P1 / 2
+//   s', within 4 u of the trial's scale (search_runs)                                  4 u VMAX s' P2
+//   C and B converted, the fma: 2 u (|s' C| + |B|) for each point                      4 u (VMAX s' M2 + 2^23 L1)
+//   the reference's float sum: 14 u d2 + u A for each point (|s q| <= |diff| + |x|; the rounded differences, two
+//   products and the additions left to right)                                          28 u d2 + 2 u A
+// A and d2 in these units are A 2^b / (2 s) and that plus F. The factors of the last line are rounded up, for the
+// second point's larger d2 and the bound's own rounding. At one point every term is convex in s: between two
+// scales the bound is no larger than at one of them.
 template <int D>
-__device__ __forceinline__ float tolerance(float sp, float rs, float a, float c0, float b0, float best) {
+__host__ __device__ __forceinline__ float tolerance(float sp, float rs, float a, float c0, float b0, float best) {
     using L = ListBound<D>;
-    constexpr float U = 5.9604645e-8f;
+    constexpr float U = 5.9604645e-8f, UV = D == 8 ? 0.5f : 0.25f;        // UV = u VMAX
     const float d2 = fmaxf(a * rs + sp * c0 - b0 + best, 0.f);
-    return 1.25f * (sp * (1.5f * L::P2 + 2.f * L::M2) + (L::P1 + L::L1) + 26.f * U * d2 + 4.f * U * (sp * c0 + a * rs));
+    return 1.01f * (sp * ((0.5f + 4.f * UV) * L::P2 + 4.f * UV * L::M2) + (L::P1 + 2.f * L::L1)) + U * (32.f * d2 + 4.f * (a * rs + sp * c0));
 }
 
 // byte planes of four 24-bit integers
@@ -422,12 +428,14 @@ __device__ __forceinline__ void sums(const uint32_t (&w)[D == 8 ? 12 : 8], const
 // is scanned at the scales of its first and last trial (FINAL: at the record's final scale) and its points
 // written, EXACT where a lead is too small to be sure of. F is linear in s, so
 //   * one point best at both ends is best between them, and the bound is no larger there than the larger of
-//     the two (it is a sum of s', constants and 1 / s);
+//     the two;
 //   * with point g at the first and h at the last trial, every third point lies above the line between the
 //     second best values of the two ends. If that line passes over the crossing of g and h, it is above the
-//     better of the two all the way: the trials before the crossing take g, the others h. If it does not, the
-//     two trials at the crossing are searched as well (the run queued again with them): g and h there mean
-//     the same; anything else leaves a shorter run on one side to be searched the same way.
+//     better of the two all the way: the trials before the crossing take g, the others h. (The crossing is
+//     right to 4 u and the line to 4 u of its ends, together less than three times the bound: four times it
+//     are asked for, the bound being the largest of the two ends and the crossing.) If it does not, the two
+//     trials at the crossing are searched as well (the run queued again with them): g and h there mean the
+//     same; anything else leaves a shorter run on one side to be searched the same way.
 // A queue entry: {map entry, lane | first trial << 8 | last << 16 | (trial before the crossing + 1) << 24 | PEELED}.
 // Returns the trials (as bits) of which some point is left open (EXACT).
 template <int K, bool FINAL>
@@ -458,7 +466,7 @@ __device__ __forceinline__ uint32_t search_runs(WaveMem<K>& W, int count, const 
         }
         const uint4 meta = W.rec[o].w[D == 8 ? 3 : 2];
         const float max = __uint_as_float(meta.x), ratio = __uint_as_float(meta.y);
-        // s' of trial t: max / num to 2 u of the trial's scale
+        // s' of trial t: max / num within 4 u (3.04 over all mantissas and trials) of the scale 1 / (num / max)
         auto scaled = [&](int t) __attribute__((always_inline)) {
             const float num = trial_num<K>(t), rn = __builtin_amdgcn_rcpf(num);
             return max * __builtin_fmaf(__builtin_fmaf(-num, rn, 1.f), rn, rn) * ratio;
@@ -513,10 +521,13 @@ __device__ __forceinline__ uint32_t search_runs(WaveMem<K>& W, int count, const 
             }
         }
         const float fc0 = (float)(uint32_t)c0, fb0 = (float)b0, av = __uint_as_float(meta.z);
+        auto bound = [&](float s, float f) __attribute__((always_inline)) {
+            return tolerance<D>(s, __builtin_amdgcn_rcpf(s) * ratio, av, fc0, fb0, f);
+        };
         float tol = 0;
         bool sure[NS], all = true;
 #pragma unroll
-        for (int k = 0; k < NS; ++k) tol = fmaxf(tol, tolerance<D>(sp[k], __builtin_amdgcn_rcpf(sp[k]) * ratio, av, fc0, fb0, m1[k]));
+        for (int k = 0; k < NS; ++k) tol = fmaxf(tol, bound(sp[k], m1[k]));
 #pragma unroll
         for (int k = 0; k < NS; ++k) {
             sure[k] = m2[k] - m1[k] > tol && id[k] < Cfg<K>::PTS;
@@ -549,10 +560,11 @@ __device__ __forceinline__ uint32_t search_runs(WaveMem<K>& W, int count, const 
                         // the trial from which h is taken (a wrong one fails the tests)
                         const float x = (max * ratio * __builtin_amdgcn_rcpf(sx) - trial_num<K>(0)) * (1.f / Cfg<K>::STEP);
                         const int tx = tmax(t0 + 1, tmin(t1, (int)ceilf(fminf(fmaxf(x, -1.f), 64.f))));
-                        const float over = k * m2[0] + (1.f - k) * m2[1] - __builtin_fmaf(sx, (float)cg, -(float)bg);
-                        if (k >= 0.f && k <= 1.f && over > 2.f * tol &&
-                            (tx - 1 == t0 || __builtin_fmaf(scaled(tx - 1), dc, -db) < -tol) &&
-                            (tx == t1 || __builtin_fmaf(scaled(tx), dc, -db) > tol))
+                        const float fx = __builtin_fmaf(sx, (float)cg, -(float)bg);
+                        const float over = k * m2[0] + (1.f - k) * m2[1] - fx, tolx = fmaxf(tol, bound(sx, fx));
+                        if (k >= 0.f && k <= 1.f && over > 4.f * tolx &&
+                            (tx - 1 == t0 || __builtin_fmaf(scaled(tx - 1), dc, -db) < -tolx) &&
+                            (tx == t1 || __builtin_fmaf(scaled(tx), dc, -db) > tolx))
                             W.point[tx][o] = (uint16_t)h;
                         else
                             again = (task.y & 0xffffffu) | ((uint32_t)tx << 24);
@@ -1036,18 +1048,50 @@ int run(const QuantArgs& a, int table) {
     return 0;
 }
 
+// fn(std::integral_constant<int, K>) of a type's kind; false for other types
+template <class F>
+bool with_kind(int type, F fn) {
+    switch (type) {
+        case 16: fn(std::integral_constant<int, K_IQ2_XXS>()); return true;
+        case 17: fn(std::integral_constant<int, K_IQ2_XS>()); return true;
+        case 22: fn(std::integral_constant<int, K_IQ2_S>()); return true;
+        case 18: fn(std::integral_constant<int, K_IQ3_XXS>()); return true;
+        case 21: fn(std::integral_constant<int, K_IQ3_S>()); return true;
+    }
+    return false;
+}
+
 }  // namespace
 
 int launch_lattice(const QuantArgs& a) {
     const int t = iq_table_index(a.type);
-    switch (a.type) {
-        case 16: return run<K_IQ2_XXS>(a, t);
-        case 17: return run<K_IQ2_XS>(a, t);
-        case 22: return run<K_IQ2_S>(a, t);
-        case 18: return run<K_IQ3_XXS>(a, t);
-        case 21: return run<K_IQ3_S>(a, t);
-    }
-    return fail(SPA_ERR_TYPE, "launch_lattice: type %d", a.type);
+    int e = SPA_OK;
+    if (!with_kind(a.type, [&](auto k) { e = run<decltype(k)::value>(a, t); }))
+        return fail(SPA_ERR_TYPE, "launch_lattice: type %d", a.type);
+    return e;
 }
 
 }  // namespace spa
+
+extern "C" int spa_lattice_trials_host(int type, int trial, const float* max, int64_t n, float* id) {
+    if (n < 0 || (n > 0 && (!max || !id))) return spa::fail(SPA_ERR_ARG, "spa_lattice_trials_host: null or negative");
+    bool in_range = false;
+    const bool known = spa::with_kind(type, [&](auto k) {
+        constexpr int K = decltype(k)::value;
+        in_range = trial >= 0 && trial < spa::Cfg<K>::T;
+        for (int64_t i = 0; in_range && i < n; ++i) id[i] = spa::trial_id<K>(trial, max[i], 1.f / max[i]);
+    });
+    if (!known) return spa::fail(SPA_ERR_TYPE, "spa_lattice_trials_host: type %d", type);
+    return in_range ? SPA_OK : spa::fail(SPA_ERR_ARG, "spa_lattice_trials_host: trial %d", trial);
+}
+
+extern "C" int spa_lattice_bound_host(int type, const float* f, float* out) {
+    if (!f || !out) return spa::fail(SPA_ERR_ARG, "spa_lattice_bound_host: null");
+    const bool known = spa::with_kind(type, [&](auto k) {
+        constexpr int D = spa::Cfg<decltype(k)::value>::D;
+        using L = spa::ListBound<D>;
+        out[0] = spa::tolerance<D>(f[0], f[1], f[2], f[3], f[4], f[5]);
+        out[1] = L::L1; out[2] = L::M2; out[3] = L::P1; out[4] = L::P2;
+    });
+    return known ? SPA_OK : spa::fail(SPA_ERR_TYPE, "spa_lattice_bound_host: type %d", type);
+}

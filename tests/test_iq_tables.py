@@ -10,6 +10,8 @@ import pytest
 from seedpack_amd._lib import check, lib
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LATTICE = {0: 16, 1: 17, 3: 22, 4: 18, 5: 21}      # table -> type
+TRIALS = {16: (5, -6, 13, 0.1), 17: (5, -9, 19, 0.1), 22: (5, -9, 19, 0.1), 18: (15, -15, 31, 0.2), 21: (15, -9, 19, 0.2)}
 NAMES = ["iq2_data_0", "iq2_data_1", "iq2_data_2", "iq2_data_3", "iq3_data_0", "iq3_data_1"]
 
 
@@ -74,28 +76,60 @@ def test_spread_of_the_neighbour_lists(i, d, levels, l1, m2, p1, p2):
         top = np.maximum(top, [np.abs(p - p[0]).sum(1).max(), np.abs(q - q[0]).sum(1).max(),
                                np.abs(p[:, None] - p[None]).sum(-1).max(), np.abs(q[:, None] - q[None]).sum(-1).max()])
     assert (top <= [l1, m2, p1, p2]).all(), top
+    kernel = np.zeros(5, np.float32)
+    check(lib().spa_lattice_bound_host(LATTICE[i], np.ones(6, np.float32).ctypes.data, kernel.ctypes.data))
+    assert list(kernel[1:]) == [l1, m2, p1, p2]
     vmax = 1 << (23 if d == 8 else 22)
     assert p2 * vmax < 1 << 31 and m2 * vmax < 1 << 31 and (pts * pts).sum(1).max() * vmax < 1 << 32
 
 
-def test_trial_scales_divide_exactly():
-    """the lattice quantizers' trial scales: num / max as one remainder step on num * (1 / max) in float32, for
-    every num of the types and a sample of mantissas that holds the ends of the range. The fused steps are
-    formed in float64: the remainder is exact there, and the last sum's rounding error decides its ties"""
+def numerators(t):
+    base, lo, n, step = TRIALS[t]
+    return [np.float32(base) + np.float32(lo + k) * np.float32(step) for k in range(n)]
+
+
+@pytest.mark.parametrize("t", sorted(TRIALS))
+def test_trial_scales_divide_exactly(t):
+    """the lattice quantizers' trial scales num / max, formed as one remainder step on num * (1 / max), are the
+    float32 quotient for every mantissa of max and every num of the type"""
+    mx = (np.arange(1 << 23, dtype=np.uint32) | np.uint32(0x3F800000)).view(np.float32)
+    got = np.empty_like(mx)
+    for k, num in enumerate(numerators(t)):
+        check(lib().spa_lattice_trials_host(t, k, mx.ctypes.data, mx.size, got.ctypes.data))
+        assert np.array_equal(got, num / mx), k
+
+
+@pytest.mark.parametrize("t", sorted(TRIALS))
+def test_filter_scales_within_four_units(t):
+    """the scale that the integer filter takes, max times a reciprocal of num that one step refines, is within
+    4 * 2^-24 of 1 / (num / max) as float32 rounds it, the hardware's reciprocal up to one unit off"""
     f, d = np.float32, np.float64
-    nums = [f(5) + f(k) * f(0.1) for k in range(-9, 10)] + [f(15) + f(k) * f(0.2) for k in range(-15, 16)]
-    m = np.unique(np.concatenate([np.arange(4096), np.arange((1 << 23) - 4096, 1 << 23), np.arange(0, 1 << 23, 127)]))
-    mx = (m.astype(np.uint32) | np.uint32(0x3F800000)).view(f)
-    r = f(1) / mx
-    for num in nums:
-        q0 = num * r
-        rem = (d(num) - mx.astype(d) * q0.astype(d)).astype(f)
-        t = rem.astype(d) * r.astype(d)
-        s = q0.astype(d) + t
-        err = t - (s - q0.astype(d))                       # exact: |t| is far below |q0|
-        want = num / mx
-        # the exact sum s + err lies within half the gap to either neighbour of the quotient
-        up, dn = np.nextafter(want, f(9e9)).astype(d), np.nextafter(want, f(-9e9)).astype(d)
-        w = want.astype(d)
-        over, under = s - (w + up) / 2, s - (w + dn) / 2
-        assert ((over < 0) | ((over == 0) & (err <= 0))).all() and ((under > 0) | ((under == 0) & (err >= 0))).all()
+    mx = (np.arange(0, 1 << 23, 7, dtype=np.uint32) | np.uint32(0x3F800000)).view(f)
+    for num in numerators(t):
+        want = f(1) / (num / mx)
+        for r in (np.nextafter(f(1) / num, f(0)), f(1) / num, np.nextafter(f(1) / num, f(9))):
+            # the fused steps: exact in float64 but for a rounding far below float32's
+            rn = f(f(1 - d(num) * d(r)) * d(r) + d(r))
+            assert np.abs((mx * rn).astype(d) / want - 1).max() <= 4 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("t", sorted(TRIALS))
+def test_lead_covers_every_rounding(t):
+    """the lead the filter asks of its best point is no less than the sum of what separates the filter's values of
+    two points from the reference's float sums (the terms listed at tolerance() in csrc/quant_lattice.hip)"""
+    g = np.random.Generator(np.random.PCG64(t))
+    u, vmax = 2.0 ** -24, 2.0 ** (22 if t in (18, 21) else 23)
+    for _ in range(4000):
+        sp = np.exp2(g.uniform(-8, 4))
+        c0, a_s = vmax * g.uniform(1, 80), 2.0 ** g.uniform(20, 27)
+        b0 = g.uniform(0, 1) * (a_s + sp * c0)
+        best = -g.uniform(0, 1.2) * (a_s + sp * c0 - b0) * g.choice([0.01, 1])
+        terms = np.array([sp, 1 / sp, a_s * sp, c0, b0, best], np.float32)
+        out = np.zeros(5, np.float32)
+        check(lib().spa_lattice_bound_host(t, terms.ctypes.data, out.ctypes.data))
+        sp, rs, a, c0, b0, best = terms.astype(np.float64)
+        l1, m2, p1, p2 = out[1:].astype(np.float64)
+        d2 = max(0.0, a * rs + sp * c0 - b0 + best)
+        need = (sp * p2 / 2 + p1 + 4 * u * vmax * sp * p2 + 4 * u * (vmax * sp * m2 + 2.0 ** 23 * l1)
+                + 28 * u * d2 + 2 * u * a * rs)
+        assert out[0] >= need, terms
