@@ -163,6 +163,10 @@ int spa_lattice_bound_host(int ggml_type, const float* terms, float* out5);
 /* Blocks per rANS segment of a type: max(16, 16384 / QK) (qr.py:952-954); 0 if not a QR type. */
 int spa_qr_seg_blocks(int ggml_type);
 
+/* The part of its row (0..7) that each of n columns lies in, as the coder's contexts take it: the first 256
+ * columns, then seven equal parts (of the model, qr.py:78-377). Host memory, the code the kernels run. */
+int spa_qr_column_parts_host(const int64_t* col, int64_t n, int cols, int32_t* part);
+
 /* Device workspace bytes spa_qr_hist and spa_qr_encode need for nseg segments of the type: per
  * block slot its equality flag and a list entry (about 5 bytes per block). */
 size_t spa_qr_work_bytes(int ggml_type, int nseg);

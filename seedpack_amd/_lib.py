@@ -60,6 +60,7 @@ SIGNATURES = {
     "spa_lattice_trials_host": (c_int, [c_int, c_int, c_void_p, c_int64, c_void_p]),
     "spa_lattice_bound_host": (c_int, [c_int, c_void_p, c_void_p]),
     "spa_qr_seg_blocks": (c_int, [c_int]),
+    "spa_qr_column_parts_host": (c_int, [c_void_p, c_int64, c_int, c_void_p]),
     "spa_qr_work_bytes": (c_size_t, [c_int, c_int]),
     "spa_qr_hist": (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                             c_void_p, c_int, c_void_p, c_void_p]),

@@ -739,6 +739,12 @@ int scratch_on_device(int* dev_out, void** out) {
 
 extern "C" {
 
+int spa_qr_column_parts_host(const int64_t* col, int64_t n, int cols, int32_t* part) {
+    if (n < 0 || (n > 0 && (!col || !part))) return spa::fail(SPA_ERR_ARG, "spa_qr_column_parts_host: null or negative");
+    for (int64_t i = 0; i < n; ++i) part[i] = spa::qr::pos8(col[i], cols);
+    return SPA_OK;
+}
+
 int spa_qr_grid_h(int T, const void* F, int64_t nw, float* h, void* stream) {
     if (nw < 0) return spa::fail(SPA_ERR_ARG, "spa_qr_grid_h: negative count");
     if (!nw) return 0;

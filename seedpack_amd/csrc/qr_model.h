@@ -500,7 +500,7 @@ __device__ __forceinline__ void seed_vals8(int st, const uint8_t* sb, int64_t gw
 }
 
 // position of a weight's column in its row: the first 256 columns, then 7 parts
-__device__ __forceinline__ int pos8(int64_t col, int cols) {
+__host__ __device__ __forceinline__ int pos8(int64_t col, int cols) {
     if (cols <= 0 || col < 256) return 0;
     // col * 7 / cols as the count of the parts' starts at or below it: six compares, where the 64-bit
     // division is some hundred instructions a weight

@@ -8,6 +8,7 @@ import pytest
 from oracle import qr as oqr
 from seedpack_amd import device as dev
 from seedpack_amd import qr, synth
+from seedpack_amd._lib import check, lib
 from seedpack_amd.gpuquant import GPUQuant
 from tests.golden.qr_cases import CASES, GRID
 from tests.test_oracle_qr import case_grid, case_inputs
@@ -175,9 +176,11 @@ def test_hip_qr_decode_seed_alignment(vectors, name, shift):
 
 
 def test_column_parts_equal_the_division():
-    """the count of the parts' starts at or below a column against the definition min(6, 7 col / cols)"""
-    for cols in (257, 512, 1000, 4096, 16384, 2**31 - 1):
-        col = np.unique(np.clip(np.concatenate([np.arange(256, 20000), [k * cols // 7 + d for k in range(1, 8) for d in (-1, 0, 1)]]), 256, cols + 255))
-        c7 = 7 * col.astype(np.int64)
-        n = sum((c7 >= cols * k).astype(np.int64) for k in range(1, 7))
-        assert np.array_equal(n, np.minimum(6, c7 // cols)), cols
+    """the part of its row that a column lies in (the kernels' own code, run on the host) against the definition:
+    0 below column 256, then 1 + min(6, 7 col / cols)"""
+    for cols in (0, 255, 256, 257, 512, 1000, 4096, 16384, 2**31 - 1):
+        col = np.unique(np.clip(np.concatenate([np.arange(20000), [k * cols // 7 + d for k in range(1, 8) for d in (-1, 0, 1)]]), 0, cols + 255))
+        part = np.full(col.size, -1, np.int32)
+        check(lib().spa_qr_column_parts_host(col.ctypes.data, col.size, cols, part.ctypes.data))
+        want = np.where(col < 256, 0, 1 + np.minimum(6, 7 * col // max(cols, 1))) if cols else 0 * col
+        assert np.array_equal(part, want), cols
