@@ -532,6 +532,10 @@ int spa_r2_decode(const void* in, uint64_t in_bytes, const uint64_t* in_off, voi
                   int nseg, const int16_t* rfi, const int16_t* cfi, const int8_t* scl, const int32_t* rowmap,
                   const uint8_t* dtab, void* stream);
 
+/* The launch spa_r2_decode chooses for nseg segments on a device of `cus` compute units: segments to a workgroup
+ * and runs of that many. No device call. */
+int spa_r2_decode_grid_host(int nseg, int cus, int* per_workgroup, int* runs);
+
 /* Compact decode tables for nctx contexts (roles x 656): context c gets table remap[c] of cum
  * (257 u32 per table), or a one-symbol table when remap[c] < 0; spa_r2_dec_table_bytes() bytes per
  * context: per 128-slot bucket the u64 (symbol | cum << 8 | freq << 24) of its first slot's symbol,

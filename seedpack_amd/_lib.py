@@ -160,6 +160,7 @@ SIGNATURES = {
                               c_void_p, c_uint64, c_void_p, c_void_p]),
     "spa_r2_decode": (c_int, [c_void_p, c_uint64, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                               c_void_p, c_void_p, c_void_p, c_void_p]),
+    "spa_r2_decode_grid_host": (c_int, [c_int, c_int, ctypes.POINTER(c_int), ctypes.POINTER(c_int)]),
     "spa_r2_build_dec_tables": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p]),
     "spa_r2_dec_table_bytes": (c_uint64, []),
     "spa_r2_copy_rows": (c_int, [c_void_p, c_int, c_void_p, c_int, c_void_p]),

@@ -848,6 +848,18 @@ __global__ __launch_bounds__(256) void k_lut(const uint32_t* __restrict__ cum, i
         for (uint32_t i = cum[tb * 257 + sym]; i < cum[tb * 257 + sym + 1]; ++i) lut[((size_t)tb << pb) + i] = (uint8_t)sym;
 }
 
+// The decode's launch: segments to a workgroup, and workgroups (runs of segments) for each part. A workgroup's
+// tables and rings fill a CU's LDS, and workgroups go to the XCDs in turn whatever runs there, while a run of
+// several roles takes several of them: with a run for every CU, an XCD that gets one more than it has CUs takes a
+// second turn (2560 segments of four roles, the whole call: 24 ms on 256 workgroups, 14.2 on 200; of one role
+// 13.3 and 13.4). So 25 of 32 CUs, and more segments than those hold in rounds of them.
+void dec_grid(int nseg, int cus, int& per_wg, int& runs) {
+    const int64_t side = cus >= 2 ? (int64_t)cus * 25 / 32 : 1, hold = side * DEC_T;
+    const int64_t rounds = (nseg + hold - 1) / hold;
+    per_wg = (int)((nseg + side * rounds - 1) / (side * rounds));
+    runs = (int)(((int64_t)nseg + per_wg - 1) / per_wg);
+}
+
 }  // namespace
 }  // namespace r2
 }  // namespace spa
@@ -920,18 +932,22 @@ int spa_r2_encode(const void* dev, const void* tb, const void* sg, int nseg, con
     return SPA_OK;
 }
 
+int spa_r2_decode_grid_host(int nseg, int cus, int* per_workgroup, int* runs) {
+    if (nseg < 1 || cus < 1 || !per_workgroup || !runs) return fail(SPA_ERR_ARG, "spa_r2_decode_grid_host: segments, CUs >= 1");
+    dec_grid(nseg, cus, *per_workgroup, *runs);
+    return SPA_OK;
+}
+
 int spa_r2_decode(const void* in, uint64_t in_bytes, const uint64_t* in_off, void* dev, const void* tb, const void* sg, int nseg,
                   const int16_t* rfi, const int16_t* cfi, const int8_t* scl, const int32_t* rowmap, const uint8_t* dtab,
                   void* stream) {
     if (nseg < 0) return fail(SPA_ERR_ARG, "spa_r2_decode: negative segment count");
     if (nseg == 0) return SPA_OK;
     if (reinterpret_cast<uintptr_t>(in) & 15) return fail(SPA_ERR_ARG, "spa_r2_decode: stream not 16-byte aligned");
-    // A workgroup's tables fill a CU's LDS. Up to 200 workgroups run side by side (2560 segments took 12.0 ms
-    // on 100 to 230, 19.9 ms on 240 and 21.4 ms on 256, where some CUs are given two while others idle); more
-    // segments than those hold go in rounds of them.
-    constexpr int SIDE = 200;
-    const int rounds = (nseg + SIDE * DEC_T - 1) / (SIDE * DEC_T);
-    const int per_wg = (nseg + SIDE * rounds - 1) / (SIDE * rounds), nrun = (nseg + per_wg - 1) / per_wg;
+    int device = 0, cus = 0, per_wg = 0, nrun = 0;
+    SPA_HIP_TRY(hipGetDevice(&device));
+    SPA_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+    dec_grid(nseg, cus, per_wg, nrun);
     hipLaunchKernelGGL(k_dec, dim3((unsigned)(nrun * DEC_PARTS)), dim3((unsigned)((per_wg + 63) / 64 * 64)), 0, (hipStream_t)stream,
                        (const uint8_t*)in, (in_bytes + 15) / 16, in_off, (uint8_t*)dev, (const TB*)tb, (const SG*)sg, nseg, per_wg,
                        nrun, rfi, cfi, scl, rowmap, dtab);

@@ -299,3 +299,20 @@ def test_hip_r2_decode_workgroups_of_several_roles(spread):
     host = np.frombuffer(data, np.uint8)
     for off, nb, _, _ in layout["t"]:
         assert out[off:off + nb].tobytes() == host[off:off + nb].tobytes()
+
+
+@pytest.mark.parametrize("n", [13_500, 104_000])
+def test_hip_r2_decode_several_waves_and_rounds(n):
+    """more segments than 200 workgroups of one wave hold, and more than their 512 lanes hold: one-row tensors of
+    six roles in turn, 8 or 9 weights each, a few of them longer than what the reader's ring holds"""
+    say("case r2 waves and rounds", n)
+    g = np.random.Generator(np.random.PCG64(n))
+    rl = np.where(np.arange(n) % 977 == 5, 300, 8 + (np.arange(n) % 7 == 3))
+    w = synth.bf16_bits((g.standard_normal(int(rl.sum())) * 0.02).astype(np.float32))
+    at = np.concatenate([[0], np.cumsum(rl)])
+    ts = [(f"blk.{i}.role{i % 6}.weight", int(2 * at[i]), int(2 * rl[i]), int(rl[i])) for i in range(n)]
+    layout = r2.layout_of(ts, w.nbytes)
+    codec = r2.BF16v2(group_bytes=1 << 30)
+    parts = codec.compress(w.tobytes(), layout)
+    assert len(parts["arrays"]["lens"]) >= n
+    assert codec.decompress(parts).tobytes() == w.tobytes()

@@ -1,12 +1,15 @@
 """Host side of the R2 codec that runs without a GPU: the chunk framing, the file's other bytes
 (rest_of / fill_rest) and both header forms (the P form also against the reference's own output in
 tests/test_archive_host.py)."""
+import ctypes
 import lzma
 import struct
 
 import numpy as np
+import pytest
 
 from seedpack_amd import framing, header
+from seedpack_amd._lib import check, lib
 
 
 def _gguf_strings(items):
@@ -81,3 +84,18 @@ def test_header_pairs_form_rebuilds_the_token_arrays():
     comp = [lzma.compress(x) for x in (stripped, lens.tobytes(), b"".join(raw), planes.tobytes())]
     buf = b"P" + struct.pack("<6Q", t0, t1, m0, m1, len(toks), len(pairs)) + struct.pack("<4I", *map(len, comp)) + b"".join(comp)
     assert header.header_d(buf) == rest
+
+
+@pytest.mark.parametrize("cus", [1, 8, 32, 64, 128, 256, 304])
+def test_decode_launch_fits_the_device(cus):
+    """every segment has a lane, a workgroup at most 512; up to a device full of them, no more runs than CUs, with
+    room beside them for the other roles of runs that hold several; more segments in the least number of rounds"""
+    side = max(1, cus * 25 // 32)
+    for n in (1, 2, 63, 64, 65, side - 1, side, side + 1, 64 * side + 1, 512 * side, 512 * side + 1, 5120 * side - 7, 2**31 - 1):
+        if n < 1:
+            continue
+        per, runs = ctypes.c_int(), ctypes.c_int()
+        check(lib().spa_r2_decode_grid_host(n, cus, ctypes.byref(per), ctypes.byref(runs)))
+        assert 1 <= per.value <= 512 and (runs.value - 1) * per.value < n <= runs.value * per.value, n
+        assert runs.value <= side * -(-n // (512 * side)), n
+    assert lib().spa_r2_decode_grid_host(0, 256, ctypes.byref(per), ctypes.byref(runs)) == -4
