@@ -603,6 +603,19 @@ def stream_buffer(n):
     return dev.DeviceArray(max(16, -(-n // 16) * 16), np.uint8)
 
 
+def by_role(roles, segs, in_off):
+    """the tensors' segments and their stream offsets, one role after another (tensor order within a role):
+    the decoder's workgroups hold one role's tables at a time, so a run of segments in file order, where
+    small tensors of many roles alternate, would be decoded role by role (2400 segments of 12 roles in
+    turn 148 ms, 13760 of 80 blocks' 7 roles 53 ms, 20608 of 28 blocks' 43 ms; in this order 58, 24, 24)"""
+    at = np.concatenate([[0], np.cumsum([len(x) for x in segs])]).astype(np.int64)
+    order = sorted(range(len(segs)), key=roles.__getitem__)
+    if not order:
+        return np.zeros(0, SG_DT), np.zeros(0, np.uint64)
+    return (np.concatenate([segs[k] for k in order]),
+            np.concatenate([np.asarray(in_off[at[k]:at[k + 1]], np.uint64) for k in order]))
+
+
 class _Decoder:
     """the decode side's tables and maps (bf16v2.py:425-451, :496-530): side information, compact
     decode tables and remap on the device, segment lengths and stream offsets, duplicate rows"""
@@ -681,9 +694,9 @@ class _Decoder:
             sg["i0"] = np.arange(0, n, SEG)
             sg["n"] = np.minimum(SEG, n - sg["i0"])
             segs.append(sg)
-        sg = np.concatenate(segs) if segs else np.zeros(0, SG_DT)
-        if len(in_off) != len(sg):
+        if len(in_off) != sum(map(len, segs)):
             raise ValueError("R2: segment offsets do not match the tensors")
+        sg, in_off = by_role([self.layout["role"][i] for i in idxs], segs, in_off)
         keep = [dev.DeviceArray.from_host(np.ascontiguousarray(in_off, np.uint64) if len(sg) else np.zeros(1, np.uint64), st),
                 dev.DeviceArray.from_host(tb.view(np.uint8) if len(tb) else np.zeros(32, np.uint8), st),
                 dev.DeviceArray.from_host(sg.view(np.uint8) if len(sg) else np.zeros(16, np.uint8), st)]

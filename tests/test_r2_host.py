@@ -8,7 +8,7 @@ import struct
 import numpy as np
 import pytest
 
-from seedpack_amd import framing, header
+from seedpack_amd import framing, header, r2
 from seedpack_amd._lib import check, lib
 
 
@@ -99,3 +99,24 @@ def test_decode_launch_fits_the_device(cus):
         assert 1 <= per.value <= 512 and (runs.value - 1) * per.value < n <= runs.value * per.value, n
         assert runs.value <= side * -(-n // (512 * side)), n
     assert lib().spa_r2_decode_grid_host(0, 256, ctypes.byref(per), ctypes.byref(runs)) == -4
+
+
+def test_decoder_takes_segments_role_by_role():
+    """tensors of several roles in turn: each role's segments side by side, in file order, each with its own
+    stream offset"""
+    g = np.random.default_rng(8)
+    roles = [int(x) for x in g.integers(0, 5, 40)]
+    segs, off, at = [], [], 1000
+    for k in range(40):
+        sg = np.zeros(int(g.integers(0, 6)), r2.SG_DT)
+        sg["t"], sg["i0"], sg["n"] = k, r2.SEG * np.arange(len(sg)), r2.SEG
+        segs.append(sg)
+        off += [at + 7 * j for j in range(len(sg))]
+        at += 7 * len(sg) + 1
+    where = {(int(s["t"]), int(s["i0"])): o for s, o in zip(np.concatenate(segs), off)}
+    sg, in_off = r2.by_role(roles, segs, np.array(off, np.uint64))
+    assert [where[int(s["t"]), int(s["i0"])] for s in sg] == [int(x) for x in in_off] and len(sg) == len(off)
+    keys = [(roles[s["t"]], int(s["t"]), int(s["i0"])) for s in sg]
+    assert keys == sorted(keys)
+    sg, in_off = r2.by_role([], [], np.zeros(0, np.uint64))
+    assert len(sg) == len(in_off) == 0
