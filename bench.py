@@ -15,8 +15,10 @@ same JSON line.
 import argparse
 import collections
 import concurrent.futures
+import hashlib
 import json
 import os
+import re
 import sys
 import threading
 import time
@@ -116,13 +118,39 @@ def cpu_baseline(tensors, target_s=12.0, type_s=1.5):
                                                 "oracle's numpy restatement (kind: port), one core"}
 
 
+def _kernel_sources(kernel):
+    """the sources that a kernel of the profiles' summaries is built from"""
+    own = {"Q8_0": "quant_legacy.hip", "Q4_0": "quant_legacy.hip", "IQ4_XS": "quant_iq4.hip", "IQ1_S": "quant_iq1.hip",
+           "IQ1_M": "quant_iq1.hip"}.get(kernel, "quant_lattice.hip" if kernel.startswith("IQ") else "quant_k.hip")
+    tables = ["iq_tables.h"] if own in ("quant_iq1.hip", "quant_lattice.hip") else []
+    return [os.path.join(ROOT, "seedpack_amd", "csrc", f) for f in [own, "common.h", "search.h"] + tables]
+
+
+def source_digest(kernel):
+    """a digest of those sources without their comments and white space"""
+    h = hashlib.sha256()
+    for p in _kernel_sources(kernel):
+        text = re.sub(r"//[^\n]*|/\*.*?\*/", "", open(p).read(), flags=re.S)
+        h.update("".join(text.split()).encode() + b"\0")
+    return h.hexdigest()[:16]
+
+
+def _profiled(name, section, kernel):
+    """a kernel's entry of a counter summary in profiles/, None if there is none or if it was counted on other
+    sources than the tree holds now: an old count over a new launch time is no measurement"""
+    p = os.path.join(ROOT, "profiles", name)
+    if not os.path.exists(p):
+        return None
+    d = json.load(open(p))
+    if d.get("sources", {}).get(kernel) != source_digest(kernel):
+        return None
+    return d.get(section, {}).get(kernel)
+
+
 def _profiled_traffic(kernel):
     """HBM bytes per launch of a kernel on the embedding, from the rocprofv3 FETCH_SIZE/WRITE_SIZE
     passes summarised in profiles/ (scaled by the copy-kernel factors recorded there)"""
-    p = os.path.join(ROOT, "profiles", "traffic.json")
-    if not os.path.exists(p):
-        return None
-    return json.load(open(p))["bytes_per_launch"].get(kernel)
+    return _profiled("traffic.json", "bytes_per_launch", kernel)
 
 
 SIMDS, CLOCK_GHZ = 1024, 2.4
@@ -165,20 +193,14 @@ def valu_probe(stream, reps=5):
 def _profiled_valu(kernel):
     """VALU lane-ops per launch of a kernel on the embedding: SQ_INSTS_VALU x 64 from the rocprofv3
     counter pass summarised in profiles/"""
-    p = os.path.join(ROOT, "profiles", "valu.json")
-    if not os.path.exists(p):
-        return None
-    d = json.load(open(p))
-    n = d["insts_valu_per_launch"].get(kernel)
-    return None if n is None else n * d["lane_ops_per_instruction"]
+    n = _profiled("valu.json", "insts_valu_per_launch", kernel)
+    return None if n is None else n * 64
 
 
 def _profiled_issue(kernel):
     """share of the SIMDs' quad-cycles issuing at least one VALU instruction, from the counter pass"""
-    p = os.path.join(ROOT, "profiles", "valu.json")
-    if not os.path.exists(p):
-        return None
-    return json.load(open(p)).get("issue", {}).get(kernel, {}).get("issue_slot_occupancy")
+    e = _profiled("valu.json", "issue", kernel)
+    return None if e is None else e["issue_slot_occupancy"]
 
 
 def _cpu_model():
@@ -798,7 +820,7 @@ def main():
                     "valu_lane_ops_per_launch": ops, "avg_launch_ms": round(dom_ms, 4), "hbm": hbm,
                     "issue_slot_occupancy": _profiled_issue(kname), "single_issue_peak": probe["single_issue_T_lane_ops_s"],
                     "frac_of_fp32_tflops": round(va / 157.3, 4), "valu_probe": probe,
-                    "note": "lane-ops = SQ_INSTS_VALU x 64 per launch (exact: profiles/valu.json) over the live launch time; "
+                    "note": "lane-ops = SQ_INSTS_VALU x 64 per launch (profiles/valu.json, counted on the same kernel source) over the live launch time; "
                             "peak = 2 x the single-issue rate the VALU probe measures in this run (spa_valu_probe: "
                             "plain 32-bit loops, no dual issue); issue_slot_occupancy = quad-cycles issuing at least "
                             "one VALU instruction (SQ_ACTIVE_INST_VALU - SQ_ACTIVE_INST_VALU2 over the SIMDs' "
@@ -806,7 +828,7 @@ def main():
                             "against the published 157.3 TFLOP/s (packed FP32, FMA = 2)"}
     else:
         roofline = {"bound": "hbm", "kernel": kdesc, **hbm, "traffic": traffic, "avg_launch_ms": round(dom_ms, 4),
-                    "note": "no VALU count profiled for this launch: HBM fraction only"}
+                    "note": "no VALU count profiled for this launch on the kernel as it is: HBM fraction only"}
 
     # HBM-bound legacy types: configuration 1 tensor and the embedding, Q8_0 / Q4_0 without imatrix
     legacy = {}
