@@ -21,15 +21,17 @@
 // its first strict minimum winning as in the C code: a few lanes' lists one after another, each by the whole
 // wave (exact_neighbour), more of them cut into pieces that are dealt to the lanes (dealt_neighbours).
 //
-// Bound by VALU issue. With the importance matrix, against one list search per trial and group: IQ2_XS
-// 4096 x 12288 6.10 to 3.14 ms (7231 to about 2450 lane-instructions a weight), IQ3_XXS 2053 x 3584 1.157
-// to 0.638 ms; on 4096 x 4096 IQ2_XXS 1.38 to 0.92 ms, IQ2_S 0.68 to 0.50 ms, IQ3_S 1.24 to 0.76 ms.
+// The SIMDs issue VALU instructions in 83-88% of their quad-cycles, almost never two at once: half of the issue
+// limit. With the importance matrix, against one list search per trial and group: IQ2_XS 4096 x 12288 6.10 to
+// 3.15 ms (7231 to 2473 lane-instructions a weight), IQ3_XXS 2053 x 3584 1.157 to 0.64 ms; on 4096 x 4096 IQ2_XXS
+// 1.48 to 0.94 ms, IQ2_S 0.75 to 0.57 ms, IQ3_S 1.29 to 0.88 ms.
 // Weights on a coarse grid, where equal distances are common, need the float sums for up to half of their trials.
 // Without the importance matrix, 4096 x 4096, us: one list search per trial and group; undecided lists one after
 // another, each by the whole wave; dealt, up to four trials at once:
 //   4-bit codes, a scale per 32    IQ2_S 712 / 3790 / 945    IQ3_XXS 1835 / 5220 / 1790    IQ3_S 1290 / 3150 / 1290
 //   three values, a scale per 128  IQ2_S 556 / 2600 / 584    IQ3_XXS 1600 / 15460 / 1490   IQ3_S  885 / 2960 /  785
-// On normal weights the dealt search, which runs there now and then, and its registers cost 1% to 2%, IQ2_S 4%.
+// On normal weights the dealt search, which runs there now and then, its registers and the bound cost 1% to 2%,
+// IQ2_S 3%.
 //
 // Mapping: one lane per sub-block (32 or 16 weights), G = 256/N lanes per super-block, 256-lane
 // workgroups, held to three waves per SIMD (8 to 212 bytes of scratch a lane; at two or four waves the kernels
@@ -50,11 +52,14 @@ constexpr int WG = 256;
 constexpr float FLT_BIG = 3.402823466e+38F;   // FLT_MAX
 constexpr uint32_t PREV = 0xffffu;            // a trial's point: that of the trial before it
 constexpr uint32_t EXACT = 0xfffeu;           // a trial's point: still to be found by the float sums
-// Open points of at most FEW lanes and FEW_TRIALS trials are found one after another, more of them dealt. (FEW = 0,
-// 2, 6: IQ2_S with normal weights 631, 606, 606 us; 6 is 10-25% slower where weights are on a fine grid.) A run that
-// is undecided at both ends is left open at once where more than MANY runs searched side by side are undecided;
-// elsewhere a near miss of one or two trials is likelier, which a further scan of the run costs less.
-constexpr int FEW = 2, FEW_TRIALS = 4, MANY = 6;
+// Open points of at most FEW lanes and FEW_TRIALS trials are found one after another, more of them dealt (FEW = 0,
+// 2, 6: IQ2_S with normal weights 631, 606, 606 us; 6 is 10-25% slower where weights are on a fine grid).
+// A run that is undecided at both ends is left open at once where more than MANY of those searched side by side
+// are undecided; so is one that is undecided once more, there and without an importance matrix, where equal weights
+// make equal distances common. Elsewhere a near miss of one or two trials is likelier, which a further scan of the run
+// costs less (left open: IQ2_XS and IQ2_S with normal weights 1% and 2% slower; scanned again without a matrix:
+// weights of three values 14-27% slower).
+constexpr int FEW = 2, FEW_TRIALS = 4, MANY = 3;
 constexpr int QCAP = 256;                     // runs a wave queues before it searches them
 constexpr uint32_t PEELED = 1u << 31;         // a queued run: what is left of one with an undecided end
 
@@ -437,9 +442,9 @@ __device__ __forceinline__ void sums(const uint32_t (&w)[D == 8 ? 12 : 8], const
 //     trials at the crossing are searched as well (the run queued again with them): g and h there mean the
 //     same; anything else leaves a shorter run on one side to be searched the same way.
 // A queue entry: {map entry, lane | first trial << 8 | last << 16 | (trial before the crossing + 1) << 24 | PEELED}.
-// Returns the trials (as bits) of which some point is left open (EXACT).
+// `ties`: no importance matrix (see MANY). Returns the trials (as bits) of which some point is left open (EXACT).
 template <int K, bool FINAL>
-__device__ __forceinline__ uint32_t search_runs(WaveMem<K>& W, int count, const Point<Cfg<K>::D>* pts, const uint16_t* __restrict__ nb) {
+__device__ __forceinline__ uint32_t search_runs(WaveMem<K>& W, int count, bool ties, const Point<Cfg<K>::D>* pts, const uint16_t* __restrict__ nb) {
     constexpr int D = Cfg<K>::D, NS = FINAL ? 1 : 2, R = Cfg<K>::R;
     const int lane = (int)__lane_id();
     uint32_t open = 0;
@@ -561,14 +566,14 @@ __device__ __forceinline__ uint32_t search_runs(WaveMem<K>& W, int count, const 
                         const float x = (max * ratio * __builtin_amdgcn_rcpf(sx) - trial_num<K>(0)) * (1.f / Cfg<K>::STEP);
                         const int tx = tmax(t0 + 1, tmin(t1, (int)ceilf(fminf(fmaxf(x, -1.f), 64.f))));
                         const float fx = __builtin_fmaf(sx, (float)cg, -(float)bg);
-                        const float over = k * m2[0] + (1.f - k) * m2[1] - fx, tolx = fmaxf(tol, bound(sx, fx));
+                        const float over = k * m2[0] + (1.f - k) * m2[1] - fx, tolx = over > 4.f * tol ? fmaxf(tol, bound(sx, fx)) : tol;
                         if (k >= 0.f && k <= 1.f && over > 4.f * tolx &&
                             (tx - 1 == t0 || __builtin_fmaf(scaled(tx - 1), dc, -db) < -tolx) &&
                             (tx == t1 || __builtin_fmaf(scaled(tx), dc, -db) > tolx))
                             W.point[tx][o] = (uint16_t)h;
                         else
                             again = (task.y & 0xffffffu) | ((uint32_t)tx << 24);
-                    } else if (task.y & PEELED || (many && !sure[0] && !sure[NS - 1])) {
+                    } else if ((task.y & PEELED && (many || ties)) || (many && !sure[0] && !sure[NS - 1])) {
                         // undecided once more, or at both ends in many lanes: equal distances, which last
                         leave_open(t0, t1);
                     } else {
@@ -845,7 +850,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(3))) void k_
             if (n > QCAP - 64 || !__ballot(left != 0)) {
                 wave_lds_sync();
                 n = sort_runs<K>(W, n, tab.map);
-                open |= search_runs<K, false>(W, n, pts, tab.nb);
+                open |= search_runs<K, false>(W, n, !imx, pts, tab.nb);
                 n = 0;
             }
         }
@@ -932,7 +937,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(3))) void k_
         if (off && filter) W.queue[lanes_below(m)] = make_uint2((uint32_t)u, (uint32_t)lane);
         wave_lds_sync();
         const int n = sort_runs<K>(W, __popcll(m), tab.map);
-        search_runs<K, true>(W, n, pts, tab.nb);
+        search_runs<K, true>(W, n, !imx, pts, tab.nb);
         settle(true, 0, xval, v, redo ? scale : 1 / bid, u);
         const int p = W.point[0][lane];
         W.best[k][lane] = (uint16_t)p;
