@@ -1,7 +1,7 @@
 """Regrow benchmark: bit-exact requantization of BF16 weights (with the imatrix) on one MI355X.
 
 A step is one pass of the hot path over one batch of synthetic input: the configuration-2 workload
-(BASELINE.json configs[1]) -- the K-quant family Q2_K, Q3_K, Q4_K, Q5_K, Q6_K with an imatrix, on
+-- the K-quant family Q2_K, Q3_K, Q4_K, Q5_K, Q6_K with an imatrix, on
 the two Qwen3-0.6B-shaped BF16 tensors token_embd 151936x1024 and ffn_down 1024x3072 (10 launches
 per step, inputs resident in HBM before timing starts).
 

@@ -476,15 +476,15 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(Cfg<K>::WPE)
     static_assert(2 * N <= (int)sizeof(Park), "a sub-block's 16-bit values fit a park slot");
     __shared__ uint4 stash[WG];
     const bool raw16 = kind != SRC_F32;
-            const uint64_t eo = (uint64_t)(sbc * 256 + sub * N);
-            stash[threadIdx.x] = make_uint4((uint32_t)eo, (uint32_t)(eo >> 32), (uint32_t)((sbc % sbpr) * 256 + sub * N),
-                                            __float_as_uint(sigma2));
-            if (raw16) {
-                const uint4* p = reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(src) + eo);
-                uint4* slot = reinterpret_cast<uint4*>(&park[lsb][sub]);
-    #pragma unroll
-                for (int k = 0; k < N / 8; ++k) slot[k] = p[k];
-            }
+    const uint64_t eo = (uint64_t)(sbc * 256 + sub * N);
+    stash[threadIdx.x] = make_uint4((uint32_t)eo, (uint32_t)(eo >> 32), (uint32_t)((sbc % sbpr) * 256 + sub * N),
+                                    __float_as_uint(sigma2));
+    if (raw16) {
+        const uint4* p = reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(src) + eo);
+        uint4* slot = reinterpret_cast<uint4*>(&park[lsb][sub]);
+#pragma unroll
+        for (int k = 0; k < N / 8; ++k) slot[k] = p[k];
+    }
     auto reload = [&](float (&xv)[N], float (&wv)[N]) {
         const uint4 st = stash[tid()];
         if (raw16) {

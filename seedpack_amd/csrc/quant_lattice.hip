@@ -21,9 +21,9 @@
 // its first strict minimum winning as in the C code: a few lanes' lists one after another, each by the whole
 // wave (exact_neighbour), more of them cut into pieces that are dealt to the lanes (dealt_neighbours).
 //
-// The SIMDs issue VALU instructions in 83-88% of their quad-cycles, almost never two at once: half of the issue
+// The SIMDs issue VALU instructions in 84-89% of their quad-cycles, almost never two at once: half of the issue
 // limit. With the importance matrix, against one list search per trial and group: IQ2_XS 4096 x 12288 6.10 to
-// 3.15 ms (7231 to 2473 lane-instructions a weight), IQ3_XXS 2053 x 3584 1.157 to 0.64 ms; on 4096 x 4096 IQ2_XXS
+// 3.18 ms (7231 to 2459 lane-instructions a weight), IQ3_XXS 2053 x 3584 1.157 to 0.64 ms; on 4096 x 4096 IQ2_XXS
 // 1.48 to 0.94 ms, IQ2_S 0.75 to 0.57 ms, IQ3_S 1.29 to 0.88 ms.
 // Weights on a coarse grid, where equal distances are common, need the float sums for up to half of their trials.
 // Without the importance matrix, 4096 x 4096, us: one list search per trial and group; undecided lists one after

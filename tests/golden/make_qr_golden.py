@@ -4,14 +4,14 @@ C++ with -ffp-contract=off, launches run on host threads). Run in the build cont
 
     python tests/golden/make_qr_golden.py
 
-Nothing here runs on the GPU box or at test time: the output is data (qr_vectors.npz).
+Nothing here runs on a GPU or at test time: the output is data (qr_vectors.npz).
 
 The kernel text is read from qr.py with `ast` (qr.py itself imports zstandard and numba, which are
 absent); `normalize` (qr.py:904-923) is taken the same way and run on numpy. The host-side steps of
 qr.encode/decode (qr.py:957-968 _layout, :1007-1090) are restated below, minus the zstd framing.
 Inputs: seeded BF16 tensors (seed type 30), predictions P = the reference quantizer's bytes
-(oracle/_ref), files F = P with 1% of blocks perturbed (one byte or nibble changed), as in
-BASELINE.json configs[0].
+(oracle/_ref), files F = P with 1% of blocks perturbed (one byte or nibble changed), as in the
+first benchmark configuration.
 """
 import ast
 import os

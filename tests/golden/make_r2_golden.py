@@ -11,7 +11,7 @@ bf16v2.py and gpu2.py import numba / zstandard (absent here), so the functions a
 are read with `ast` and executed against the --cpu backend; the driver steps of
 BF16v2._analyse / _encode (bf16v2.py:323-411: per group of tensors, statistics, dedup, histogram;
 normalisation; encode, gather) are restated below without the GGUF parsing and header coding.
-Nothing here runs on the GPU box or at test time: the output is data (r2_vectors.npz).
+Nothing here runs on a GPU or at test time: the output is data (r2_vectors.npz).
 """
 import argparse
 import ast
